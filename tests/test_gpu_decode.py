@@ -151,3 +151,65 @@ def test_seventeen_rows_stay_on_the_prefill_kernel():
     out = abi.attn_fwd(q, k, v, 0.0625, False)
     torch.cuda.synchronize()
     assert orc.max_abs_err(out.cpu(), _oracle(q, k, v, 0.0625)) <= TOL["bf16"]
+
+
+MASKED = [
+    # dtype, B, H, Hkv, Sq, Sk, D, mask
+    ("bf16", 3, 8, 2, 1, 1000, 128, "pad_bool"),       # rows 4-byte aligned: a dword of 4 keys per lane
+    ("bf16", 3, 8, 2, 1, 3001, 128, "pad_bool"),       # odd rows: an element at a time; split, empty parts
+    ("fp16", 2, 8, 8, 1, 77, 64, "pad_bool"),          # one row per unit, a ragged last tile
+    ("fp16", 1, 8, 2, 4, 515, 96, "rows_bool"),        # 16 packed rows, a mask of their own each
+    ("bf16", 2, 6, 2, 2, 1030, 160, "heads_bf16"),     # additive, per query head (packed rows), -inf runs
+    ("fp16", 2, 4, 4, 5, 333, 192, "rows_f16"),
+    ("bf16", 1, 16, 1, 1, 9001, 256, "rows_f32"),      # one unit, deep split merged in two levels
+    ("fp16", 1, 4, 4, 16, 40, 224, "offset_bool"),     # a base off 4 bytes, one part
+    ("bf16", 40, 8, 8, 1, 260, 128, "pad_bool"),       # more units than CUs: no split
+]
+
+
+def _decode_mask(kind, B, H, Sq, Sk, seed):
+    """The last query row of the last batch entry sees no key (zeros)."""
+    g = torch.Generator().manual_seed(seed)
+    if kind == "pad_bool":
+        m = torch.ones(B, 1, 1, Sk, dtype=torch.bool)
+        for b in range(B):
+            m[b, ..., :b * Sk // (2 * B)] = False
+        m[-1] = False
+        return m.cuda()
+    if kind == "offset_bool":
+        buf = torch.rand(Sq * Sk + 3, generator=g) > 0.5
+        buf[3 + (Sq - 1) * Sk:] = False
+        return buf.cuda()[3:].view(1, 1, Sq, Sk)
+    if kind == "rows_bool":
+        m = torch.rand(B, 1, Sq, Sk, generator=g) > 0.7
+        m[-1, :, -1] = False
+        return m.cuda()
+    m = torch.randn(B if "rows" in kind else 1, H, Sq, Sk, generator=g) * 2
+    m[..., : Sk // 3] = -math.inf
+    m[..., -1, Sk // 2:] = torch.finfo(torch.float16).min  # finite, far below the rest
+    m[-1, :, -1] = -math.inf
+    return m.to({"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[kind.split("_")[1]]).cuda()
+
+
+@pytest.mark.parametrize("case", MASKED, ids=[f"{c[0]}-b{c[1]}h{c[2]}of{c[3]}-q{c[4]}k{c[5]}d{c[6]}-{c[7]}" for c in MASKED])
+def test_masked_decode(case):
+    """Masked decode steps: query heads packed per K/V head, each packed row
+    with its own mask row; split and unsplit launches meet the oracle, rows
+    that see no key are zeros, and reruns are bit-identical."""
+    dtype, B, H, Hkv, Sq, Sk, D, kind = case
+    print(f"masked decode {case}", flush=True)
+    q, k, v = _inputs(dtype, B, H, Hkv, Sq, Sk, D, seed=Sk + D)
+    m = _decode_mask(kind, B, H, Sq, Sk, seed=Sk)
+    scale = 1.0 / math.sqrt(D)
+    split1, split2, whole = torch.empty_like(q), torch.empty_like(q), torch.empty_like(q)
+    assert abi.attn_fwd_raw(q, k, v, split1, scale, False, attn_mask=m) == 0
+    assert abi.attn_fwd_raw(q, k, v, split2, scale, False, attn_mask=m) == 0
+    assert abi.attn_fwd_raw(q, k, v, whole, scale, False, attn_mask=m, workspace=False) == 0
+    torch.cuda.synchronize()
+    g = H // Hkv
+    want = orc.sdpa_np(q.cpu(), k.cpu().repeat_interleave(g, dim=1), v.cpu().repeat_interleave(g, dim=1), scale,
+                       False, attn_mask=m.cpu())
+    assert torch.equal(split1, split2)
+    for out in (split1, whole):
+        assert orc.max_abs_err(out.cpu(), want) <= TOL[dtype]
+        assert not out[-1, :, -1].any()

@@ -36,6 +36,7 @@ struct FwdParams {
   // {batch, head, query}; unit stride along keys; kind: MASK_* below
   const void* mask;
   int64_t m_b, m_h, m_q;
+  int64_t m_g;  // packed grouped-query rows: mask stride of one query head (m_h: a group of them)
   int mask_kind;
   // the mask is read element by element, nothing past key Sk - 1 of a row
   // (any layout with unit key stride); otherwise in runs of 8 keys, every
@@ -46,7 +47,7 @@ struct FwdParams {
   // row's scale * Q K^T over its visible keys (what a backward pass needs to
   // rebuild P); null = not written.  Written by the pipelined kernel only.
   float* lse;
-  // grouped-query row packing (pipelined kernel, non-causal): when pack_sq > 0
+  // grouped-query row packing (non-causal): when pack_sq > 0
   // the launch runs over K/V heads, and row r of head hk is query position
   // r % pack_sq of query head hk * G + r / pack_sq; q_h / o_h then step over a
   // whole group of query heads and q_g / o_g over one query head
@@ -220,6 +221,19 @@ __device__ __forceinline__ void lds_dma16(const u32x4& rs, uint32_t lds_byte, in
 // lds_dma16; used for the small per-tile slices of attention masks).
 __device__ __forceinline__ void lds_dma4(const u32x4& rs, uint32_t lds_byte, int voff, int soff) {
   asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
+               ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds_byte)
+               : "memory");
+}
+
+// 1 or 2 bytes per lane, zero-extended to 4 bytes in LDS at lds_byte + 4 i
+// (as lds_dma4; attention masks whose rows are not 4-byte aligned).
+__device__ __forceinline__ void lds_dma1(const u32x4& rs, uint32_t lds_byte, int voff, int soff) {
+  asm volatile("s_nop 0\n\tbuffer_load_ubyte %0, %1, %2 offen lds"
+               ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds_byte)
+               : "memory");
+}
+__device__ __forceinline__ void lds_dma2(const u32x4& rs, uint32_t lds_byte, int voff, int soff) {
+  asm volatile("s_nop 0\n\tbuffer_load_ushort %0, %1, %2 offen lds"
                ::"v"(voff), "s"(rs), "s"(soff), "{m0}"(lds_byte)
                : "memory");
 }

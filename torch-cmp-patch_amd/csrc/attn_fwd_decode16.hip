@@ -1,5 +1,6 @@
-// Decode-step attention forward for fp16 / bf16 on gfx950: few query rows per
-// K/V head (a decode step, or a short speculative block), a long key sweep.
+// Decode-step attention forward for fp16 / bf16 on gfx950, masked or not: few
+// query rows per K/V head (a decode step, or a short speculative block), a long
+// key sweep.
 //
 // Such a launch moves almost nothing but K and V (B * H_kv heads of Sk rows
 // each, read once), so it is bound by how many bytes the chip keeps in flight
@@ -136,7 +137,13 @@ __device__ __forceinline__ int64_t dec_row(int r, int pack_sq, int64_t g_str, in
   return (int64_t)r * s_str;
 }
 
-template <typename T, int DK>
+// MK: mask loads per lane and tile (0: no mask).  A lane's scores of a tile
+// are 4 consecutive keys of one row; their mask elements ride the wave's ring
+// beside K and V, so that no ordinary load stands between the DMA loads that
+// vmcnt counts (the compiler's own wait for it would drain them).  MK = 1: a
+// bool mask whose rows are 4-byte aligned, one dword; MK = 4: any kind and
+// alignment, one element each.
+template <typename T, int DK, int MK>
 __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p, DecArgs a) {
   constexpr int NS = dec_stages(DK);
   constexpr int RB = DK * 2;            // bytes of a K/V row in LDS
@@ -149,13 +156,15 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
   constexpr int DQ = DK / 4;            // float4 vectors of an output row
   static_assert(DK % 32 == 0 && DK >= 64 && DK <= 256, "head dim");
   static_assert(BLK % 1024 == 0, "a block is whole DMA instructions");
-  static_assert(2 * IB * (NS - 1) <= 63, "vmcnt range");
+  constexpr int IPT = 2 * IB + MK;      // DMA instructions per tile
+  constexpr int MSLOT = MK * 256;       // bytes of a tile's mask elements
+  static_assert(IPT * (NS - 1) <= 63, "vmcnt range");
   constexpr int MOS = DK + 4;           // row stride (floats) of the waves' merge rows
   static_assert(kDecNw * kDecRows * MOS * 4 + 2 * kDecNw * kDecRows * 4 + 16 <= kDecNw * NS * STAGE,
                 "the workgroup's merge fits in the ring's LDS");
   static_assert(2 * kDecRows * kDecMaxParts * 4 + 2 * kDecRows * 4 + 16 + kDecNw * 64 * 16 <= kDecNw * NS * STAGE,
                 "the parts' merge fits in the ring's LDS");
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kDecNw * NS * STAGE];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kDecNw * NS * (STAGE + MSLOT)];
 
   const int tid = thread_x(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -220,6 +229,47 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
   const uint32_t ring = lds0 + (uint32_t)(wave * NS * STAGE);
   const u32x4 krw = uniform_rsrc_words(kg, ((int64_t)(Sk - 1) * p.k_s + D) * 2);
   const u32x4 vrw = uniform_rsrc_words(vg, ((int64_t)(Sk - 1) * p.v_s + D) * 2);
+  // mask of this unit's rows; row c (rows past R read the last one) at byte
+  // mrow, keys past Sk at an offset beyond the buffer (nothing is read)
+  const int mes = p.mask_kind == MASK_BOOL ? 1 : p.mask_kind == MASK_F32 ? 4 : 2;
+  const uint32_t mring = lds0 + (uint32_t)(kDecNw * NS * STAGE + wave * NS * MSLOT);
+  u32x4 mrw = {0u, 0u, 0u, 0u};
+  int mrow = 0;
+  if constexpr (MK > 0) {
+    mrow = (int)dec_row(min(c, R - 1), p.pack_sq, p.m_g, p.m_q) * mes;
+    const int64_t last = dec_row(R - 1, p.pack_sq, p.m_g, p.m_q);
+    mrw = uniform_rsrc_words((const char*)p.mask + (b * p.m_b + hk * p.m_h) * mes, (last + Sk) * mes);
+  }
+  auto issue_mask = [&](int j, int key0) {
+    const uint32_t ms = mring + (uint32_t)((j % NS) * MSLOT);
+#pragma unroll
+    for (int e = 0; e < MK; ++e) {
+      const int vo = key0 + 4 * g + e < Sk ? mrow + (4 * g + e) * mes : (int)0x80000000u;
+      if (MK == 1 || mes == 4) lds_dma4(mrw, ms + 256 * e, vo, key0 * mes);
+      else if (mes == 2) lds_dma2(mrw, ms + 256 * e, vo, key0 * mes);
+      else lds_dma1(mrw, ms + 256 * e, vo, key0 * mes);
+    }
+  };
+  // a tile's mask (stage j % NS) applied to this lane's exp2-domain scores
+  auto apply_mask = [&](int j, float (&x)[4]) {
+    const unsigned char* ms = lds + kDecNw * NS * STAGE + (wave * NS + j % NS) * MSLOT + 4 * lane;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t w = *(const uint32_t*)(ms + (MK == 1 ? 0 : 256 * e));
+      if (p.mask_kind == MASK_BOOL) {
+        if ((MK == 1 ? (w >> (8 * e)) & 0xffu : w) == 0u) x[e] = -INFINITY;
+      } else {
+        const float f = p.mask_kind == MASK_F32   ? __uint_as_float(w)
+                        : p.mask_kind == MASK_F16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)w)
+                                                  : __uint_as_float(w << 16);
+        x[e] = __builtin_fmaf(f, kLog2e, x[e]);
+      }
+    }
+  };
+  // weight of a state whose offset is m against the offset mx; with a mask a
+  // row may have seen no key (m = -inf): weight 0
+  auto weight = [&](float m, float mx) { return MK > 0 && m == -INFINITY ? 0.f : fast_exp2(m - mx); };
+  auto inverse = [&](float l) { return MK > 0 && !(l > 0.f) ? 0.f : 1.f / l; };
   // this wave's tile j into stage j % NS (rows past Sk read zeros)
   auto issue = [&](int j) {
     const int key0 = (t0 + wave + kDecNw * j) * kDecBk;
@@ -229,6 +279,7 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
     for (int i = 0; i < IB; ++i) lds_dma16(krw, st + 1024 * i, kdo[i], sk);
 #pragma unroll
     for (int i = 0; i < IB; ++i) lds_dma16(vrw, st + BLK + 1024 * i, vdo[i], sv);
+    if constexpr (MK > 0) issue_mask(j, key0);
   };
 
   f32x4 oacc[NDB];
@@ -245,9 +296,9 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
     // tile j has landed once at most (tiles still in flight behind it) x
     // (instructions per tile) loads are outstanding
     const int behind = min(NS - 1, mine - 1 - j);
-    if (behind >= 3) wait_vmcnt<6 * IB>();
-    else if (behind == 2) wait_vmcnt<4 * IB>();
-    else if (behind == 1) wait_vmcnt<2 * IB>();
+    if (behind >= 3) wait_vmcnt<3 * IPT>();
+    else if (behind == 2) wait_vmcnt<2 * IPT>();
+    else if (behind == 1) wait_vmcnt<IPT>();
     else wait_vmcnt<0>();
     const unsigned char* st = lds + (wave * NS + j % NS) * STAGE;
     const int key0 = (t0 + wave + kDecNw * j) * kDecBk;
@@ -264,20 +315,30 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[e] = key0 + 4 * g + e < Sk ? s[e] * cmul : -INFINITY;
     }
+    if constexpr (MK > 0) {  // the mask first, so that keys past Sk stay out whatever it holds
+      apply_mask(j, x);
+      if (key0 + kDecBk > Sk) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (key0 + 4 * g + e >= Sk) x[e] = -INFINITY;
+      }
+    }
     float mt = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
     mt = fmaxf(mt, shfl_xor_f(mt, 16));
     mt = fmaxf(mt, shfl_xor_f(mt, 32));
     if (__builtin_amdgcn_ballot_w64(mt > m_run)) {  // some row's maximum rises
       const float m_new = fmaxf(m_run, mt);
-      const float alpha = fast_exp2(m_run - m_new);  // 0 on the first tile (m_run = -inf)
+      // 0 on the row's first tile (m_run = -inf), or until it sees a key (O and l are 0 then)
+      const float alpha = weight(m_run, m_new);
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
       for (int db = 0; db < NDB; ++db) oacc[db] *= alpha;
     }
+    const float m_sub = MK > 0 && m_run == -INFINITY ? 0.f : m_run;
     u32x2 pb;
-    pb[0] = Dec<T>::pack(fast_exp2(x[0] - m_run), fast_exp2(x[1] - m_run));
-    pb[1] = Dec<T>::pack(fast_exp2(x[2] - m_run), fast_exp2(x[3] - m_run));
+    pb[0] = Dec<T>::pack(fast_exp2(x[0] - m_sub), fast_exp2(x[1] - m_sub));
+    pb[1] = Dec<T>::pack(fast_exp2(x[2] - m_sub), fast_exp2(x[3] - m_sub));
     l_run = Dec<T>::sum2(pb[1], Dec<T>::sum2(pb[0], l_run));  // the rounded P the PV MFMA takes
 
     const uint16_t* vs = (const uint16_t*)(st + BLK);
@@ -341,7 +402,7 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
       o += *(const f32x4*)(mo + (w * kDecRows + r) * MOS + 4 * k) * f;
     }
     if (nparts == 1) {
-      store_out(r, k, o, 1.f / l);
+      store_out(r, k, o, inverse(l));
     } else {
       // device-scope (aux 16 = sc1) stores, coherent across the XCDs' L2s
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), wsr, slot(part, r, k), 0, 16);
@@ -401,15 +462,15 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
       float* const wr = wq + r * n;
       const float* const lr = lq + r * n;
       float mx = -INFINITY;
-      for (int j = lane; j < n; j += 64) mx = fmaxf(mx, wr[j]);  // every part has keys: finite
+      for (int j = lane; j < n; j += 64) mx = fmaxf(mx, wr[j]);  // every part has keys: finite, without a mask
 #pragma unroll
       for (int m = 32; m >= 1; m >>= 1) mx = fmaxf(mx, shfl_xor_f(mx, m));
       float L = 0.f;
-      for (int j = lane; j < n; j += 64) L = __builtin_fmaf(lr[j], fast_exp2(wr[j] - mx), L);
+      for (int j = lane; j < n; j += 64) L = __builtin_fmaf(lr[j], weight(wr[j], mx), L);
 #pragma unroll
       for (int m = 32; m >= 1; m >>= 1) L += shfl_xor_f(L, m);
-      const float inv = fin ? 1.f / L : 1.f;
-      for (int j = lane; j < n; j += 64) wr[j] = fast_exp2(wr[j] - mx) * inv;  // this lane's own entries
+      const float inv = fin ? inverse(L) : 1.f;
+      for (int j = lane; j < n; j += 64) wr[j] = weight(wr[j], mx) * inv;  // this lane's own entries
       if (!fin && lane == 0) {
         rt[2 * r] = mx;
         rt[2 * r + 1] = L;
@@ -476,7 +537,16 @@ __global__ __launch_bounds__(kDecNw * 64, 1) void attn_fwd_decode16(FwdParams p,
 
 template <typename T, int DK>
 hipError_t launch_dk(const FwdParams& p, const DecArgs& a, int units, hipStream_t s) {
-  hipLaunchKernelGGL((attn_fwd_decode16<T, DK>), dim3(units * a.parts), dim3(kDecNw * 64), 0, s, p, a);
+  const dim3 grid(units * a.parts), block(kDecNw * 64);
+  // one mask dword per lane and tile where every group of 4 keys is 4-byte
+  // aligned and inside its row, else an element at a time
+  const int64_t align = (int64_t)(uintptr_t)p.mask | p.m_b | p.m_h | p.m_g | p.m_q | p.Sk;
+  if (p.mask_kind == MASK_NONE)
+    hipLaunchKernelGGL((attn_fwd_decode16<T, DK, 0>), grid, block, 0, s, p, a);
+  else if (p.mask_kind == MASK_BOOL && align % 4 == 0)
+    hipLaunchKernelGGL((attn_fwd_decode16<T, DK, 1>), grid, block, 0, s, p, a);
+  else
+    hipLaunchKernelGGL((attn_fwd_decode16<T, DK, 4>), grid, block, 0, s, p, a);
   return hipGetLastError();
 }
 
@@ -496,27 +566,36 @@ hipError_t launch_t(const FwdParams& p, const DecArgs& a, int units, hipStream_t
 
 }  // namespace
 
-bool packs_query_heads(const FwdParams& p, bool causal);
+bool packs_query_heads(const FwdParams& p, bool causal, bool masked_rows);
 void pack_query_heads(FwdParams& p);
 
 // Head dims of this kernel: whole 32-column score steps, 64 to 256.
 static bool decode16_dim(int D) { return D % 32 == 0 && D >= 64 && D <= 256; }
 
-// True when a launch is a decode shape this kernel takes: non-causal,
-// unmasked inference with whole aligned 16-byte chunks, at most 16 query rows
-// per K/V head once grouped query heads are packed, key rows that do not
-// overlap (rows past Sk then lie past the buffer and read zeros) and every
-// tile addressable with 32-bit buffer offsets.  Up to D = 128 the pipelined
-// kernel's decode path is as fast while the units (batch x K/V heads) fill
-// half the CUs or more (within 2-4% either way on MI355X); below that its key
-// split cuts deeper and this kernel's merge wins (1.4-2x at 8 units).
+// True when a launch is a decode shape this kernel takes: non-causal
+// inference with whole aligned 16-byte chunks, at most 16 query rows per K/V
+// head once grouped query heads are packed, key rows that do not overlap (rows
+// past Sk then lie past the buffer and read zeros) and every tile and mask
+// element addressable with 32-bit buffer offsets.  Up to D = 128 the pipelined
+// kernel's unmasked decode path is as fast while the units (batch x K/V heads)
+// fill half the CUs or more (within 2-4% either way on MI355X); below that its
+// key split cuts deeper and this kernel's merge wins (1.4-2x at 8 units).  Its
+// masked path neither packs query heads nor spares the rowless waves' work, so
+// masked steps come here whatever their units (bf16 [8,32/8,1,3001,128] with a
+// bool key-padding mask, 64 units: 301 us there, 27 us here, 3.6 TB/s).
 bool decode16_applies(const FwdParams& p, bool causal) {
-  if (causal || p.mask_kind != MASK_NONE || p.lse || p.elem_rows || !decode16_dim(p.D)) return false;
-  const bool packs = packs_query_heads(p, causal);
+  if (causal || p.lse || p.elem_rows || !decode16_dim(p.D)) return false;
+  const bool masked = p.mask_kind != MASK_NONE;
+  const bool packs = packs_query_heads(p, causal, masked);
   const int64_t rows = packs ? (int64_t)p.kv_group * p.Sq : p.Sq;
   if (rows > kDecRows) return false;
   const int64_t units = (int64_t)p.B * (packs ? p.H / p.kv_group : p.H);
-  if (p.D <= 128 && 2 * units >= device_cus()) return false;
+  if (!masked && p.D <= 128 && 2 * units >= device_cus()) return false;
+  if (masked) {
+    const int64_t mes = p.mask_kind == MASK_BOOL ? 1 : p.mask_kind == MASK_F32 ? 4 : 2;
+    const int64_t last = (packs ? (p.kv_group - 1) * p.m_h : 0) + (p.Sq - 1) * p.m_q;
+    if ((last + p.Sk + kDecBk) * mes >= INT32_MAX) return false;
+  }
   const int64_t ks = p.Sk > 1 ? p.k_s : p.D, vs = p.Sk > 1 ? p.v_s : p.D;
   if (ks < p.D || vs < p.D) return false;
   return (int64_t)(p.Sk + kDecBk) * (ks > vs ? ks : vs) * 2 < (int64_t)INT32_MAX;
@@ -570,7 +649,7 @@ int dec_group(int parts, int rows, int D) {
 
 hipError_t launch_decode16(const FwdParams& p0, bool bf16, hipStream_t s) {
   FwdParams p = p0;
-  if (packs_query_heads(p, false)) pack_query_heads(p);
+  if (packs_query_heads(p, false, true)) pack_query_heads(p);
   if (p.Sk == 1) p.k_s = p.v_s = p.D;  // one row: rows past it must lie past the buffer
   const int units = p.B * p.H;
   if (units == 0) return hipSuccess;

@@ -88,7 +88,7 @@ hipError_t launch_short16(const FwdParams& p, int dk, bool bf16, hipStream_t s);
 void describe_short16(int dk, int Sq, int Sk, char* buf, int len);
 hipError_t launch_pipe16(const FwdParams& p, int dk, bool bf16, bool causal, bool prescale, hipStream_t s);
 void describe_pipe16(int dk, int B, int H, int Sq, int Sk, bool causal, bool narrow, char* buf, int len);
-bool packs_query_heads(const FwdParams& p, bool causal);
+bool packs_query_heads(const FwdParams& p, bool causal, bool masked_rows);
 void pack_query_heads(FwdParams& p);
 bool decode16_applies(const FwdParams& p, bool causal);
 hipError_t launch_decode16(const FwdParams& p, bool bf16, hipStream_t s);
@@ -122,7 +122,7 @@ hipError_t launch_mfma16(const FwdParams& p0, bool bf16, bool causal, hipStream_
   // over K/V heads with the group's query rows packed into one problem (the
   // pipelined kernel packs for itself)
   FwdParams p = p0;
-  const bool pack = packs_query_heads(p0, causal) && !short16_applies(p0, dk, causal) &&
+  const bool pack = packs_query_heads(p0, causal, false) && !short16_applies(p0, dk, causal) &&
                     !((!p0.elem_rows || p0.elem_rows >= 4) && pipe16_applies(p0, dk));
   if (pack) pack_query_heads(p);
   if (p.elem_rows) {

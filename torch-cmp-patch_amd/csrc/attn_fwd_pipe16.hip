@@ -391,12 +391,14 @@ bool pipe16_applies(const FwdParams& p, int dk) {
 // Grouped-query launches whose query heads hold less than one block of rows
 // each (decode, short prefills) pack the G query heads of a K/V head into the
 // rows of one problem: the K/V of that head is then streamed once for all of
-// them, instead of once per query head with mostly empty blocks.  Non-causal,
-// unmasked, inference launches only (the row position then does not matter).
+// them, instead of once per query head with mostly empty blocks.  Non-causal
+// inference launches only (the row position then does not matter), unmasked
+// unless the kernel reads the mask by packed row (masked_rows: the decode
+// kernel).
 constexpr int kPackMaxSq = 64;
 
-bool packs_query_heads(const FwdParams& p, bool causal) {
-  return !causal && p.kv_group > 1 && p.Sq <= kPackMaxSq && p.mask_kind == MASK_NONE && !p.lse &&
+bool packs_query_heads(const FwdParams& p, bool causal, bool masked_rows) {
+  return !causal && p.kv_group > 1 && p.Sq <= kPackMaxSq && (masked_rows || p.mask_kind == MASK_NONE) && !p.lse &&
          p.pack_sq == 0 && (int64_t)p.kv_group * p.Sq <= (int64_t)INT32_MAX / 2;
 }
 
@@ -405,6 +407,8 @@ void pack_query_heads(FwdParams& p) {
   p.pack_sq = p.Sq;
   p.q_g = p.q_h;
   p.o_g = p.o_h;
+  p.m_g = p.m_h;
+  p.m_h *= G;
   p.q_h *= G;  // packed head hk starts at query head hk * G
   p.o_h *= G;
   p.H /= G;
@@ -414,7 +418,7 @@ void pack_query_heads(FwdParams& p) {
 
 hipError_t launch_pipe16(const FwdParams& p0, int dk0, bool bf16, bool causal, bool prescale, hipStream_t s) {
   FwdParams p = p0;
-  if (packs_query_heads(p, causal)) pack_query_heads(p);
+  if (packs_query_heads(p, causal, false)) pack_query_heads(p);
   // the training forward and the narrow-row variants have the 64 and 128
   // buckets only up to D = 128; above it the training forward has 192 and
   // 256, and neither it nor masked launches pre-scale Q (one instantiation
