@@ -200,6 +200,19 @@ size_t cmpext3_attn_fwd_workspace_size(int dtype, int B, int H, int H_kv, int Sq
                                        int mask_dtype, int causal, int with_lse);
 
 /*
+ * Bytes beyond cmpext3_attn_fwd_workspace_size (or, where that is 0, beyond
+ * CMPEXT3_WORKSPACE_COUNTER_BYTES) with which cmpext3_attn_fwd_ws first brings
+ * this bool mask (strides as passed there) into bit form on the device: the
+ * launch then loads no mask elements and leaves out the key tiles a query
+ * block keeps no key of.  One bit per mask element (dimensions of stride 0
+ * once) and a byte per 128 rows x 32 keys.  0 when the launch has no use for
+ * it.  With less workspace the mask is read as it is: the same result within
+ * rounding.  Host-only.
+ */
+size_t cmpext3_attn_fwd_mask_workspace_size(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D,
+                                            int mask_dtype, const int64_t mask_str[3], int causal);
+
+/*
  * The key split a launch of this problem (contiguous [B,H,S,D] tensors) takes
  * with workspace_bytes of workspace: *key_parts receives the key ranges each
  * split query block is cut into (1 = unsplit; 0 on error).  Returns the code

@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libcmpext3_
 # Every function include/cmpext3_attn.h declares.
 SYMBOLS = ("cmpext3_attn_fwd", "cmpext3_attn_fwd_gqa", "cmpext3_attn_fwd_masked",
            "cmpext3_attn_fwd_ws", "cmpext3_attn_fwd_workspace_size", "cmpext3_attn_fwd_plan",
+           "cmpext3_attn_fwd_mask_workspace_size",
            "cmpext3_attn_fwd_noalloc", "cmpext3_attn_fwd_lse", "cmpext3_attn_bwd",
            "cmpext3_attn_bwd_ws", "cmpext3_attn_bwd_workspace_size",
            "cmpext3_attn_strerror", "cmpext3_attn_abi_version", "cmpext3_attn_describe")
@@ -56,6 +57,8 @@ def lib() -> ctypes.CDLL:
         L.cmpext3_attn_fwd_ws.restype = ci
         L.cmpext3_attn_fwd_workspace_size.argtypes = [ci] * 10
         L.cmpext3_attn_fwd_workspace_size.restype = sz
+        L.cmpext3_attn_fwd_mask_workspace_size.argtypes = [ci] * 8 + [i64p, ci]
+        L.cmpext3_attn_fwd_mask_workspace_size.restype = sz
         L.cmpext3_attn_fwd_plan.argtypes = [ci] * 10 + [sz, ctypes.POINTER(ci)]
         L.cmpext3_attn_fwd_plan.restype = ci
         L.cmpext3_attn_fwd_lse.argtypes = [vp, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci, ci,
@@ -95,6 +98,13 @@ def workspace_size(dtype: int, B: int, H: int, Hkv: int, Sq: int, Sk: int, D: in
     """Bytes of workspace the full key-split plan of this problem takes (host only)."""
     return lib().cmpext3_attn_fwd_workspace_size(dtype, B, H, Hkv, Sq, Sk, D, mask_dtype,
                                                  int(causal), int(with_lse))
+
+
+def mask_workspace_size(dtype: int, B: int, H: int, Hkv: int, Sq: int, Sk: int, D: int,
+                        mask_dtype: int, mask_strides, causal: bool = False) -> int:
+    """Bytes beyond workspace_size that a bool mask's bit form takes (host only)."""
+    return lib().cmpext3_attn_fwd_mask_workspace_size(dtype, B, H, Hkv, Sq, Sk, D, mask_dtype,
+                                                      (ctypes.c_int64 * 3)(*mask_strides), int(causal))
 
 
 def plan(dtype: int, B: int, H: int, Hkv: int, Sq: int, Sk: int, D: int, workspace_bytes: int,
@@ -188,8 +198,9 @@ def attn_fwd_raw(q, k, v, o, scale: float, causal: bool = False, stream=None,
     mp, mdt, mst, _keep = _mask_args(attn_mask, B, H, Sq, k.shape[2])
     wp, wb = None, 0
     if workspace is True and q.is_cuda:
-        wp, wb = workspace_for(q, handle, workspace_size(dt, B, H, k.shape[1], Sq, k.shape[2], Dx,
-                                                         mdt, causal))
+        need = workspace_size(dt, B, H, k.shape[1], Sq, k.shape[2], Dx, mdt, causal)
+        bits = mask_workspace_size(dt, B, H, k.shape[1], Sq, k.shape[2], Dx, mdt, mst, causal)
+        wp, wb = workspace_for(q, handle, max(need, WORKSPACE_COUNTER_BYTES) + bits if bits else need)
     elif workspace is not False and workspace is not None:
         wp, wb = workspace.data_ptr(), workspace.numel()
     return lib().cmpext3_attn_fwd_ws(*ptrs, dt, B, H, k.shape[1], Sq, k.shape[2], Dx, *strides,

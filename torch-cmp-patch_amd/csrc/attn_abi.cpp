@@ -29,6 +29,7 @@ BwdSplit bwd_split(int dtype, int B, int H, int Hkv, int Sq, int Sk, int D, bool
 hipError_t launch_bwd32(const BwdParams& p, bool causal, hipStream_t s);
 hipError_t launch_mfma16(const FwdParams& p, bool bf16, bool causal, hipStream_t s);
 hipError_t launch_mfma32(const FwdParams& p, bool causal, hipStream_t s);
+bool decode16_applies(const FwdParams& p, bool causal);
 int mfma16_bucket(int D);
 int mfma32_bucket(int D);
 void describe_mfma16(int D, int B, int H, int Sq, int Sk, bool causal, bool bf16, char* buf, int len);
@@ -342,6 +343,26 @@ size_t cmpext3_attn_fwd_workspace_size(int dtype, int B, int H, int H_kv, int Sq
       need = info.need;
   }
   return need;
+}
+
+size_t cmpext3_attn_fwd_mask_workspace_size(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D,
+                                            int mask_dtype, const int64_t mask_str[3], int causal) {
+  if (check_shape(dtype, B, H, Sq, Sk, D) != CMPEXT3_OK || (int64_t)B * H * Sq == 0) return 0;
+  if (dtype == CMPEXT3_DTYPE_F32 || mask_dtype != CMPEXT3_DTYPE_BOOL || !mask_str) return 0;
+  if (H_kv < 1 || H_kv > H || H % H_kv != 0) return 0;
+  cmpext3::FwdParams p;
+  memset(&p, 0, sizeof p);
+  p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.D = D;
+  p.kv_group = H / H_kv;
+  p.mask_kind = cmpext3::MASK_BOOL;
+  p.m_b = mask_str[0]; p.m_h = mask_str[1]; p.m_q = mask_str[2];
+  p.k_s = p.v_s = (D + 7) / 8 * 8;
+  p.mask_narrow = 1;  // the layout with the most use for it
+  cmpext3::MaskBits mb;
+  if (!cmpext3::mask_bits_applies(p, causal != 0) || cmpext3::decode16_applies(p, causal != 0) ||
+      !cmpext3::mask_bits_plan(p, &mb))
+    return 0;
+  return mb.bytes + 256;  // the exchange in front of it ends anywhere
 }
 
 int cmpext3_attn_fwd_plan(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D, int mask_dtype,

@@ -43,6 +43,14 @@ struct FwdParams {
   // row readable up to Sk rounded up to 8 (16-byte aligned base, strides a
   // multiple of 4 elements, Sk a multiple of 8)
   int mask_narrow;
+  // the bool mask in bit form (attn_fwd_mask_bits.hip), null when not made:
+  // words [32-key tile][row] and tile classes [128-row block][tile] of each
+  // (batch, head); strides 0 over dimensions the mask broadcasts over
+  const uint32_t* bits;
+  const unsigned char* bit_cls;
+  int64_t bits_b, bits_h;  // words
+  int64_t cls_b, cls_h;    // bytes
+  int bit_rows;            // mask rows: Sq, or 1 for all queries
   // optional [B*H, Sq] fp32 output: natural-log log-sum-exp of each query
   // row's scale * Q K^T over its visible keys (what a backward pass needs to
   // rebuild P); null = not written.  Written by the pipelined kernel only.
@@ -324,6 +332,20 @@ constexpr int split_vectors(int dp) { return dp / 8 + 1; }
 constexpr int kExchangeCounters = 16384;  // CMPEXT3_WORKSPACE_COUNTER_BYTES / 4
 constexpr size_t kExchangeCounterBytes = kExchangeCounters * sizeof(int);
 
+// Bool mask to bit form (attn_fwd_mask_bits.hip): mask pointer and strides,
+// the shape of the result (dimensions broadcast over have size 1) and where
+// it goes.
+struct MaskBits {
+  const void* mask;
+  int64_t m_b, m_h, m_q;
+  int batch, heads, rows, Sk, nt;  // nt: 32-key tiles
+  uint32_t* words;
+  unsigned char* cls;
+  size_t words_bytes, bytes;       // of the words, and of words and classes
+};
+constexpr int kMaskBitsMaxTiles = 2048;  // a block's tile list sits in LDS
+constexpr int64_t kMaskBitsMaxBytes = int64_t(128) << 20;
+
 // What a launch would do (FwdParams::dry): the workspace bytes that let its
 // full key-split plan run (0: it never splits) and the key ranges per split
 // block it takes with the workspace it was given (1: unsplit).
@@ -332,7 +354,7 @@ struct SplitInfo {
   int parts;
 };
 
-// Bind a key-split plan to exchange space (host side, attn_fwd_pipe16.hip).
+// Bind a key-split plan to exchange space (host side, attn_fwd_plan16.hip).
 // The plan cuts each of its split blocks into `parts` key ranges; one range
 // of all of them takes part_bytes of partials and the plan uses ncnt
 // counters.  Returns the key ranges that fit the space FwdParams names (the
@@ -341,6 +363,13 @@ struct SplitInfo {
 // records the full plan's need and the part count in p.dry and binds
 // nothing.
 int bind_exchange(const FwdParams& p, int parts, size_t part_bytes, int ncnt, f32x4** ws, int** cnt);
+
+// Shape and size of the bit form of p's mask (false: not a bool mask, or past
+// the limits above), whether a launch would use one, and the pass that makes
+// it.
+bool mask_bits_plan(const FwdParams& p, MaskBits* a);
+bool mask_bits_applies(const FwdParams& p, bool causal);
+hipError_t launch_mask_bits(const MaskBits& a, hipStream_t s);
 
 // Raw buffer resource over [base, base + bytes) (gfx9 dword3: 32-bit raw
 // reads).  The fields go through readfirstlane so that the compiler keeps the

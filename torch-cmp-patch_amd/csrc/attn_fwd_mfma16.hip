@@ -1,7 +1,7 @@
 // Instantiations and tile table of the fp16/bf16 MFMA attention kernel
 // (kernel template in attn_fwd_mfma16.h), and the fp16/bf16 entry point:
 // head dims up to 128, and unmasked inference prefills above 128, go to the
-// software-pipelined kernel (attn_fwd_pipe16.hip); the other launches above
+// software-pipelined kernel (attn_fwd_pipe16.h); the other launches above
 // 128 (masked, training, few query rows, short key sweeps), and K/V row
 // strides too large for its 32-bit buffer offsets, run this one.
 //

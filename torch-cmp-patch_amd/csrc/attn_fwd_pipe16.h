@@ -77,6 +77,12 @@ namespace cmpext3 {
 // and 8): the mask is the same for every query row (m_q = 0, or one row)
 // and read in whole runs: wave 0 loads each tile's slice of the mask row
 // into a ring beside K, and the waves read it from LDS after the barrier.
+// OPT bit 11 (with bit 8, without bit 4): a bool mask in bit form
+// (FwdParams::bits).  The block's sweep runs over the list of tiles in which
+// some pair of the block is kept, made in LDS from the tile classes at the
+// start; each wave brings its 32 rows' words of a tile into a ring beside K,
+// and tiles of class 2 (every pair kept) are not touched.
+//
 // One workgroup's work on one query block: key tiles [g.tbase, g.tbase +
 // g.ntiles) of block (g.bh, g.qblk).  With g.nparts > 1 that is key range
 // g.part of the block's g.nparts, exchanged through row g.sb of the exchange
@@ -84,6 +90,10 @@ namespace cmpext3 {
 struct Pipe16Seg {
   int bh, qblk, part, nparts, pstride, sb, tbase, ntiles;
 };
+// Tile list entries (OPT bit 11): a tile index, with flags for a tile none of
+// whose pairs count (filling up a list shorter than the parts) and for one
+// that needs no mask.
+constexpr int kTileDead = 0x8000, kTileFull = 0x4000;
 
 template <typename T, int DK, int DP, int NW, int BK, int OCC, bool CAUSAL, bool PRESCALE, int OPT = 0>
 __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitArgs& sa, const Pipe16Seg& g) {
@@ -92,6 +102,7 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
   constexpr bool SWZ = (OPT & 2) && (DK == DP) && (DK == 32 || DK == 64 || DK == 128);
   constexpr bool MASK = (OPT & 16) != 0;
   constexpr bool NARROW = (OPT & 64) != 0;
+  constexpr bool BITS = (OPT & 2048) != 0;
   // K/V tile row strides (halves): rows padded by 16 bytes, by 48 at D = 128
   // (fewer LDS bank conflicts there: 2-3% faster on causal bf16 D = 128,
   // no change at D = 64)
@@ -124,7 +135,9 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
 
   // masked DMA launches: a ring of NR 128-byte slices of the mask, one per
   // tile (query-broadcast masks; see add_mask)
-  constexpr int MSLOT = (MASK && DMA) ? 64 : 0;  // halves per mask slice
+  constexpr int MSLOT = (MASK && DMA) ? 64 : BITS ? NW * 64 : 0;  // halves per mask slice (bits: 32 words per wave)
+  static_assert(!BITS || (DMA && !MASK && !CAUSAL && BK == 32 && NW == 4), "mask bits ride the LDS DMA ring");
+  __shared__ uint16_t tlist[BITS ? kMaskBitsMaxTiles : 1];  // this block's tiles
   __shared__ __attribute__((aligned(16))) uint16_t lds[NR * KTILE + NR * VTILE + NR * MSLOT];
   uint16_t* const kbase = lds;                // K(j) at kbase + (j % NR) * KTILE
   uint16_t* const vbase = lds + NR * KTILE;   // V(j) at vbase + (j % NR) * VTILE
@@ -162,8 +175,54 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
 
   int kend = Sk;
   if (CAUSAL) kend = min(Sk, q0 + BQ);
-  const int tbase = g.tbase, ntiles = g.ntiles;
+  int tbase = g.tbase, ntiles = g.ntiles;
+  if constexpr (BITS) {
+    // the tiles in which this block keeps a pair, in order; every wave makes
+    // the whole list (the same values) and reads back its own writes
+    const int nt = (Sk + BK - 1) / BK;
+    const unsigned char* const cls = p.bit_cls + b * p.cls_b + h * p.cls_h + (p.bit_rows > 1 ? (int64_t)qblk * nt : 0);
+    int n = 0;
+    for (int t0 = 0; t0 < nt; t0 += 256) {
+      int c[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c[i] = t0 + 64 * i + lane < nt ? cls[t0 + 64 * i + lane] : 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(c[i] != 0);
+        const int at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        if (c[i] != 0) tlist[at] = (uint16_t)((t0 + 64 * i + lane) | (c[i] == 2 ? kTileFull : 0));
+        n += __builtin_popcountll(m);
+      }
+    }
+    for (int i = n + lane; i < nparts; i += 64) tlist[i] = (uint16_t)kTileDead;  // a tile for every part
+    n = __builtin_amdgcn_readfirstlane(n < nparts ? nparts : n);
+    tbase = part * n / nparts;
+    ntiles = (part + 1) * n / nparts - tbase;
+  }
   if (ntiles <= 0) return;  // Sk == 0 is rejected by the host
+  // Tile j of this sweep.  Bits: lane l holds list entries tbase + wbase + l
+  // and + 64, which an entry is read from without a memory access; the loop
+  // moves the window on every 64 tiles.  Clamped to the last tile; past it
+  // none of its keys count.
+  int wbase = 0;
+  int wcur = 0, wnext = 0;
+  if constexpr (BITS) {
+    wcur = tlist[tbase + min(lane, ntiles - 1)];
+    wnext = tlist[tbase + min(64 + lane, ntiles - 1)];
+  }
+  auto entry = [&](int j) {
+    if constexpr (BITS) {
+      const int i = min(j, ntiles - 1) - wbase;
+      const int e = i < 64 ? __builtin_amdgcn_readlane(wcur, i) : __builtin_amdgcn_readlane(wnext, i - 64);
+      return j < ntiles ? e : (e | kTileDead);
+    } else {
+      return 0;
+    }
+  };
+  auto tile_of = [&](int j) {
+    if constexpr (BITS) return entry(j) & (kMaskBitsMaxTiles - 1);
+    else return tbase + min(j, ntiles - 1);
+  };
   // end of this workgroup's key range: the padding tile past it is masked
   const int kpe = min(kend, (tbase + ntiles) * BK);
   const int nt2 = (ntiles + 1) & ~1;  // iterations run (even)
@@ -323,13 +382,13 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
   const u32x4 vrw = uniform_rsrc_words(vg, ((int64_t)(Sk - 1) * p.v_s + D) * 2);
   // tile j (clamped to the last one) into ring slot `slot`
   auto dma_k = [&](int j, int slot) {
-    const int so = (tbase + min(j, ntiles - 1)) * BK * ks_b;
+    const int so = tile_of(j) * BK * ks_b;
 #pragma unroll
     for (int i = 0; i < DIK; ++i)
       if (64 * i + lane < SPWK) lds_dma16(krw, lds0 + 2 * (slot * KTILE + (wv * SPWK + 64 * i) * 8), dko[i], so);
   };
   auto dma_v = [&](int j, int slot) {
-    const int so = (tbase + min(j, ntiles - 1)) * BK * vs_b;
+    const int so = tile_of(j) * BK * vs_b;
 #pragma unroll
     for (int i = 0; i < DIV; ++i)
       if (64 * i + lane < SPWV)
@@ -347,7 +406,17 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
   const u32x4 mrw = uniform_rsrc_words(MASK ? (const void*)((const char*)p.mask + (b * p.m_b + h * p.m_h) * mbytes)
                                             : (const void*)p.q,
                                        MASK ? mask_span(p, mbytes) : 0);
+  // Bits: each wave brings its own 32 rows' words of tile j (rows past Sq
+  // repeat the last one: their output is never stored)
+  const u32x4 brw = uniform_rsrc_words(BITS ? (const void*)(p.bits + b * p.bits_b + h * p.bits_h) : p.q,
+                                       BITS ? (int64_t)((Sk + BK - 1) / BK) * p.bit_rows * 4 : 0);
+  const int brow = BITS && p.bit_rows > 1 ? 4 * min(qlo + lane, Sq - 1) : 0;
   auto dma_m = [&](int j, int slot) {
+    if constexpr (BITS) {
+      if (lane < 32)
+        lds_dma4(brw, lds0 + 2 * (NR * (KTILE + VTILE) + slot * MSLOT) + 128 * wv, brow, tile_of(j) * p.bit_rows * 4);
+      return;
+    }
     if (mbc && wv == 0 && lane < BK * mbytes / 4) {
       int vo = 4 * lane;
       asm volatile("" : "+v"(vo));  // computed here, not held through the loop
@@ -461,6 +530,7 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     }
   };
   auto tile_needs_mask = [&](int j) {
+    if constexpr (BITS) return (entry(j) & (kTileDead | kTileFull)) != kTileFull;
     const int k0 = (tbase + j) * BK;
     return (k0 + BK > kpe) || (CAUSAL && k0 + BK - 1 > qlo);
   };
@@ -468,6 +538,20 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
   // taken) branch: written plainly, the compiler hoists the 16 per-element key
   // computations out of the branch and every tile pays for them.
   auto mask = [&](int j, f32x16 (&sc)[NKB]) {
+    if constexpr (BITS) {
+      // this lane's row: bit 16 (r / 8) + 8 hh + r % 8 is register r's key
+      const uint32_t* const ws = (const uint32_t*)(mbase + (j & (NR - 1)) * MSLOT) + 32 * wv + l32;
+      const uint32_t w = entry(j) & kTileDead ? 0u : *ws;
+      if (__builtin_amdgcn_ballot_w64(w != 0xffffffffu)) {
+        const int x = (int)(w >> (8 * hh));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe(x, 16 * (r >> 3) + (r & 7), 1);
+          sc[0][r] = __uint_as_float((__float_as_uint(sc[0][r]) & keep) | (0xff800000u & ~keep));
+        }
+      }
+      return;
+    }
     int k0 = (tbase + j) * BK + 8 * hh;
     asm volatile("" : "+v"(k0));
 #pragma unroll
@@ -762,7 +846,7 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     // sweep (key 0 under causal; rows past Sq score 0), so that tile already
     // set the offset and thr is 8; only a mask can leave it at -inf.
     float tsum = tc0 + tc1;
-    if (__builtin_amdgcn_ballot_w64((MASK && thr == -INFINITY) || tsum > 256.f)) {
+    if (__builtin_amdgcn_ballot_w64(((MASK || BITS) && thr == -INFINITY) || tsum > 256.f)) {
       const float mx = xhalf_max(row_max(sc));
       if (__builtin_amdgcn_ballot_w64(mx > thr)) {
         const float delta = rescale(mx);
@@ -823,6 +907,13 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     // exit after an even number of iterations waits for nothing (the loads
     // write no registers)
     for (int t = 0; t < nt2; t += 4) {
+      if constexpr (BITS) {
+        if (t - wbase == 64) {  // steps t .. t + 3 reach tile t + 7
+          wbase = t;
+          wcur = wnext;
+          wnext = tlist[tbase + min(t + 64 + lane, ntiles - 1)];
+        }
+      }
       step(t, sA, sB, pA, pB, tA0, tA1, tB0, tB1, kA, vA);
       step(t + 1, sB, sA, pB, pA, tB0, tB1, tA0, tA1, kB, vB);
       if (t + 2 >= nt2) break;
@@ -1116,7 +1207,9 @@ attn_fwd_pipe16(const FwdParams p, const SplitArgs sa) {
       part = r - (lb - sa.nfull) * nparts;
     }
     int bh, qblk;
-    wg_tile(lb, p, CAUSAL, bh, qblk);
+    // a mask of its own for every query row is most often causal in shape, so
+    // its blocks start in the causal order (last block first)
+    wg_tile(lb, p, CAUSAL || ((OPT & 2048) && p.bit_rows > 1), bh, qblk);
     int kend = p.Sk;
     if (CAUSAL) kend = min(p.Sk, (qblk + 1) * NW * 32);
     const int ntall = (kend + BK - 1) / BK;

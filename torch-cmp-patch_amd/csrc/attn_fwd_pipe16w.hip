@@ -1,6 +1,6 @@
 // Instantiations of the software-pipelined fp16/bf16 kernel (template in
 // attn_fwd_pipe16.h) for head dims above 128: unmasked inference prefills of
-// the 160, 192 and 256 buckets (plan and dispatch in attn_fwd_pipe16.hip;
+// the 160, 192 and 256 buckets (plan and dispatch in attn_fwd_plan16.hip;
 // masked and training launches in attn_fwd_pipe16wm.hip).
 // One wave per SIMD (the O accumulator alone takes DK registers per lane, and
 // the compiler parks what does not fit in the accumulation registers), K/V

@@ -3,7 +3,7 @@
 // 16; buckets 160, 192, 256) or the row log-sum-exp of the training forward
 // (OPT bit 32; buckets 192 and 256, masked or not): one wave per SIMD, K/V
 // straight into LDS with padded rows, Q never pre-scaled (one instantiation
-// per dtype serves every scale).  Plan and dispatch in attn_fwd_pipe16.hip.
+// per dtype serves every scale).  Plan and dispatch in attn_fwd_plan16.hip.
 #include "attn_fwd_pipe16.h"
 
 namespace cmpext3 {

@@ -1,14 +1,6 @@
-// Instantiations, tile table and key-split plan of the software-pipelined
-// fp16/bf16 kernel (template in attn_fwd_pipe16.h), used for head dims up to
-// 128, and for the unmasked inference prefills above 128 (instantiations in
-// attn_fwd_pipe16w.hip).
-//
-// Like the v2 table in attn_fwd_mfma16.hip this replaces the reference's
-// per-head-dim template table (src/cuda/fp16_flash_attention_hfma2.cu:278-285);
-// entries come from an offline sweep on an MI355X.  All buckets use 4-wave
-// workgroups and 32-key tiles; the waves per SIMD are the most the registers
-// allow without spilling (D = 32: 4, D <= 64: 3, D <= 128: 2; above 128 one,
-// with accumulation registers as the spill space).
+// Launch plans of the software-pipelined fp16/bf16 kernel (attn_fwd_pipe16.h):
+// which problems it takes, the key split, stream-K, the bit form of bool
+// masks, and the exchange space of every split kernel.
 //
 // The key split (no counterpart in the reference) needs exchange space, and
 // the library allocates none: the workspace entry points take it from the
@@ -20,17 +12,11 @@
 
 #include <mutex>
 
-#include "attn_fwd_pipe16.h"
+#include "attn_fwd_plan16.h"
 
 namespace cmpext3 {
 
 namespace {
-
-constexpr int kPipeNw = 4;
-constexpr int kPipeBk = 32;
-constexpr int pipe_occ(int dk) { return dk <= 32 ? 4 : dk <= 64 ? 3 : dk <= 128 ? 2 : 1; }
-// masked launches need a few more registers: D = 32 drops to 3 waves per SIMD
-constexpr int pipe_occ_masked(int dk) { return dk <= 64 ? 3 : 2; }
 
 // Split plan limits: a part scans at least kMinPartTiles key tiles (shorter
 // parts spend more on their prologue and merge than they save); with no
@@ -183,134 +169,42 @@ SplitArgs streamk_plan(int n, int ntiles, int occ, int cus) {
   return sa;
 }
 
-// The mask is the same for every query row and is read in whole runs.
-bool mask_bcast(const FwdParams& p) {
-  return p.mask_kind != MASK_NONE && !p.mask_narrow && (p.m_q == 0 || p.Sq == 1);
-}
-
-template <typename T, int DK, bool CAUSAL, bool PRESCALE, int MOPT>
-hipError_t launch_dk(const FwdParams& p, const SplitArgs& sa, hipStream_t s) {
-  // OPT 1: s_setprio around the MFMA blocks; OPT 8: zero K columns past D;
-  // OPT 16 (MOPT): attention mask
-  constexpr int occ = MOPT ? pipe_occ_masked(DK) : pipe_occ(DK);
-  // OPT 128: a single query block whose last waves hold no rows (decode,
-  // packed query groups); those waves become the only K/V loaders and the
-  // waves with rows only compute.  Taken with at least two rowless waves (the
-  // loaders' chunk split assumes 128 or more loader threads); decode steps
-  // run 0-20% faster than with every wave loading and computing.
-  if constexpr (!CAUSAL && MOPT == 0) {
-    if (p.Sq <= (kPipeNw - 2) * 32) {
-      if (p.D == DK) return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 128>(p, sa, s);
-      return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 8 | 128>(p, sa, s);
-    }
-  }
-  // OPT 256 | 2: unmasked launches of the 32 / 64 / 128 buckets load K/V
-  // tiles straight into swizzled LDS (no staging registers, one load
-  // instruction per 2 KiB of tile, no bank conflicts; 3-4% faster on SDXL
-  // self-attention, 6% on causal bf16 D = 128 than register staging).
-  if constexpr (MOPT == 0 && (DK == 32 || DK == 64 || DK == 128)) {
-    // OPT 512: stream-K (equal shares of the block-tile sequence; see
-    // attn_fwd_pipe16.h), planned by launch_pipe16
-    if constexpr (!CAUSAL) {
-      if (sa.sk_wgs > 0) {
-        if (p.D == DK) return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 256 | 512>(p, sa, s);
-        return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 8 | 256 | 512>(p, sa, s);
-      }
-    }
-    if (p.D == DK) return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 256>(p, sa, s);
-    return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 8 | 256>(p, sa, s);
-  }
-  // masked launches of those buckets: the same LDS DMA, whose freed staging
-  // registers the mask words use (masked fp16 D = 64 spilled 3-21 registers
-  // with register staging; SDXL self-attention with a key-padding mask
-  // 162 -> 121 us with the mask test of attn_fwd_pipe16.h)
-  if constexpr (MOPT != 0 && (DK == 32 || DK == 64 || DK == 128)) {
-    // OPT 1024: a query-broadcast mask read in runs (key padding [B,1,1,Sk]
-    // and the like): its tile slices ride the DMA ring, no loads in the step
-    if (mask_bcast(p)) {
-      if (p.D == DK) return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 256 | 1024 | MOPT>(p, sa, s);
-      return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 8 | 256 | 1024 | MOPT>(p, sa, s);
-    }
-    if (p.D == DK) return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 256 | MOPT>(p, sa, s);
-    return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 2 | 8 | 256 | MOPT>(p, sa, s);
-  }
-  if (p.D == DK) return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | MOPT>(p, sa, s);
-  return launch_pipe16_cfg<T, DK, kPipeNw, kPipeBk, occ, CAUSAL, PRESCALE, 1 | 8 | MOPT>(p, sa, s);
-}
-
-// Training forward (OPT 32: write the row log-sum-exp; MOPT 16: with an
-// attention mask): buckets 64 and 128 only.
-template <typename T, bool CAUSAL, bool PRESCALE, int MOPT>
-hipError_t launch_lse_m(const FwdParams& p, const SplitArgs& sa, int dk, hipStream_t s) {
-  // K/V straight into swizzled LDS, as for inference; query-broadcast masks
-  // with K (OPT 1024)
-  constexpr int LD = 2 | 256;
-  if constexpr (MOPT != 0) {
-    if (mask_bcast(p)) {
-      if (dk == 64) {
-        if (p.D == 64)
-          return launch_pipe16_cfg<T, 64, kPipeNw, kPipeBk, pipe_occ(64), CAUSAL, PRESCALE, 1 | 32 | MOPT | LD | 1024>(p, sa, s);
-        return launch_pipe16_cfg<T, 64, kPipeNw, kPipeBk, pipe_occ(64), CAUSAL, PRESCALE, 1 | 8 | 32 | MOPT | LD | 1024>(p, sa, s);
-      }
-      if (dk == 128) {
-        if (p.D == 128)
-          return launch_pipe16_cfg<T, 128, kPipeNw, kPipeBk, pipe_occ(128), CAUSAL, PRESCALE, 1 | 32 | MOPT | LD | 1024>(p, sa, s);
-        return launch_pipe16_cfg<T, 128, kPipeNw, kPipeBk, pipe_occ(128), CAUSAL, PRESCALE, 1 | 8 | 32 | MOPT | LD | 1024>(p, sa, s);
-      }
-      return hipErrorNotSupported;
-    }
-  }
-  if (dk == 64) {
-    if (p.D == 64)
-      return launch_pipe16_cfg<T, 64, kPipeNw, kPipeBk, pipe_occ(64), CAUSAL, PRESCALE, 1 | 32 | MOPT | LD>(p, sa, s);
-    return launch_pipe16_cfg<T, 64, kPipeNw, kPipeBk, pipe_occ(64), CAUSAL, PRESCALE, 1 | 8 | 32 | MOPT | LD>(p, sa, s);
-  }
-  if (dk == 128) {
-    if (p.D == 128)
-      return launch_pipe16_cfg<T, 128, kPipeNw, kPipeBk, pipe_occ(128), CAUSAL, PRESCALE, 1 | 32 | MOPT | LD>(p, sa, s);
-    return launch_pipe16_cfg<T, 128, kPipeNw, kPipeBk, pipe_occ(128), CAUSAL, PRESCALE, 1 | 8 | 32 | MOPT | LD>(p, sa, s);
-  }
-  return hipErrorNotSupported;
-}
-
-template <typename T, bool CAUSAL, bool PRESCALE>
-hipError_t launch_lse(const FwdParams& p, const SplitArgs& sa, int dk, hipStream_t s) {
-  return p.mask_kind != MASK_NONE ? launch_lse_m<T, CAUSAL, PRESCALE, 16>(p, sa, dk, s)
-                                  : launch_lse_m<T, CAUSAL, PRESCALE, 0>(p, sa, dk, s);
-}
-
-// Narrow rows (OPT 64, FwdParams::elem_rows 4 or 8): inference, masked
-// (MOPT 16) or not, buckets 64 and 128 only (other head dims are zero-padded
-// up to them).
-template <typename T, bool CAUSAL, int MOPT = 0>
-hipError_t launch_narrow(const FwdParams& p, const SplitArgs& sa, int dk, hipStream_t s) {
-  constexpr int occ64 = MOPT ? pipe_occ_masked(64) : pipe_occ(64);
-  constexpr int occ128 = MOPT ? pipe_occ_masked(128) : pipe_occ(128);
-  if (dk == 64)
-    return launch_pipe16_cfg<T, 64, kPipeNw, kPipeBk, occ64, CAUSAL, false, 1 | 64 | MOPT>(p, sa, s);
-  if (dk == 128)
-    return launch_pipe16_cfg<T, 128, kPipeNw, kPipeBk, occ128, CAUSAL, false, 1 | 64 | MOPT>(p, sa, s);
-  return hipErrorNotSupported;
-}
-
-template <typename T, bool CAUSAL, bool PRESCALE, int MOPT = 0>
-hipError_t launch_bucket(const FwdParams& p, const SplitArgs& sa, int dk, hipStream_t s) {
-  switch (dk) {
-    case 32: return launch_dk<T, 32, CAUSAL, PRESCALE, MOPT>(p, sa, s);
-    case 48: return launch_dk<T, 48, CAUSAL, PRESCALE, MOPT>(p, sa, s);
-    case 64: return launch_dk<T, 64, CAUSAL, PRESCALE, MOPT>(p, sa, s);
-    case 80: return launch_dk<T, 80, CAUSAL, PRESCALE, MOPT>(p, sa, s);
-    case 96: return launch_dk<T, 96, CAUSAL, PRESCALE, MOPT>(p, sa, s);
-    case 128: return launch_dk<T, 128, CAUSAL, PRESCALE, MOPT>(p, sa, s);
-  }
-  return hipErrorNotSupported;
-}
-
-
 }  // namespace
 
-hipError_t launch_pipe16_wide(const FwdParams& p, const SplitArgs& sa, int dk, bool bf16, bool causal,
-                              bool prescale, hipStream_t s);
+// The instantiation of a planned launch up to D = 128 (narrow rows are never
+// pre-scaled).
+static hipError_t launch_pipe16_kernel(const FwdParams& p, const SplitArgs& sa, int dk, bool bf16, bool causal,
+                                       bool prescale, hipStream_t s) {
+  if (bf16) return launch_pipe16_bf16(p, sa, dk, causal, s);
+  return prescale && !p.elem_rows ? launch_pipe16_f16ps(p, sa, dk, causal, s) : launch_pipe16_f16(p, sa, dk, causal, s);
+}
+
+// A bool mask goes to bit form first (attn_fwd_mask_bits.hip) where that repays
+// the extra launch (3-4 us).  Read element by element (narrow), it does from
+// the shortest sweeps on: fp16 [2,10,4096,77,64] with a padding mask 23.4 ->
+// 15.6 us, [1,12,77,77,64] 16.8 -> 9.5, bf16 [4,16,1531,1531,128] causal and
+// padded 492 -> 61.  In whole runs: above D = 64 from 256 keys (bf16
+// [4,16/8,S,S,128] at S = 256: 24.3 -> 17.0 us causal and padded, 20.6 -> 15.6
+// key padding; at 2048: 198 -> 76 and 160 -> 141); up to D = 64 past 256 keys
+// with a row for each query ([4,32,S,S,64] at S = 256: 13.5 -> 14.4, at 288:
+// 17.5 -> 14.2), and, since one row for all queries rides the ring in runs for
+// little, with that only from 768 (at 600: 25.8 -> 27.9, at 768: 33.5 -> 32.6).
+bool mask_bits_applies(const FwdParams& p, bool causal) {
+  MaskBits a;
+  if (causal || p.lse || p.elem_rows || p.mask_kind != MASK_BOOL || !mask_bits_plan(p, &a)) return false;
+  if (p.mask_narrow) return p.Sk >= 32;
+  if (p.D > 64) return p.Sk >= 256;
+  return a.rows > 1 ? p.Sk > 256 : p.Sk >= 768;
+}
+
+// The space for a mask's bit form: behind the `used` bytes of exchange of the
+// caller's workspace (or the fixed scratch).  Null when it does not fit.
+static char* bits_space(const FwdParams& p, size_t used, size_t bytes) {
+  char* const base = p.fixed_exchange ? (char*)scratch_ptr() : (char*)p.workspace;
+  const size_t room = p.fixed_exchange ? kScratchBytes : p.workspace_bytes;
+  used = (used + 255) / 256 * 256;
+  return base && used + bytes <= room ? base + used : nullptr;
+}
 
 // Compute units of the current device (256 on MI355X), cached per device.
 int device_cus() {
@@ -445,9 +339,7 @@ hipError_t launch_pipe16(const FwdParams& p0, int dk0, bool bf16, bool causal, b
     if (p.dry) sk_need = p.dry->need;
     if (fit == sk.nparts) {
       if (p.dry) return hipSuccess;
-      return bf16 ? launch_bucket<__bf16, false, false>(p, sk, dk, s)
-                  : prescale ? launch_bucket<_Float16, false, true>(p, sk, dk, s)
-                             : launch_bucket<_Float16, false, false>(p, sk, dk, s);
+      return launch_pipe16_kernel(p, sk, dk, bf16, false, prescale, s);
     }
   }
   const int n_qblk = (p.Sq + kPipeNw * 32 - 1) / (kPipeNw * 32);
@@ -469,39 +361,30 @@ hipError_t launch_pipe16(const FwdParams& p0, int dk0, bool bf16, bool causal, b
     if (sk_need > p.dry->need) p.dry->need = sk_need;
     return hipSuccess;
   }
-  if (dk > 128) return launch_pipe16_wide(p, sa, dk, bf16, causal, prescale, s);
-  if (p.lse) {  // training forward, masked or not
-    if (bf16) return causal ? launch_lse<__bf16, true, false>(p, sa, dk, s) : launch_lse<__bf16, false, false>(p, sa, dk, s);
-    if (prescale)
-      return causal ? launch_lse<_Float16, true, true>(p, sa, dk, s) : launch_lse<_Float16, false, true>(p, sa, dk, s);
-    return causal ? launch_lse<_Float16, true, false>(p, sa, dk, s) : launch_lse<_Float16, false, false>(p, sa, dk, s);
-  }
-  if (p.elem_rows) {  // never pre-scaled: the narrow fp16 kernels then spill
-    if (p.mask_kind != MASK_NONE) {
-      if (bf16)
-        return causal ? launch_narrow<__bf16, true, 16>(p, sa, dk, s) : launch_narrow<__bf16, false, 16>(p, sa, dk, s);
-      return causal ? launch_narrow<_Float16, true, 16>(p, sa, dk, s)
-                    : launch_narrow<_Float16, false, 16>(p, sa, dk, s);
+  if (mask_bits_applies(p, causal)) {
+    MaskBits mb;
+    mask_bits_plan(p, &mb);
+    const size_t nsplit = sa.nparts > 1 ? n - sa.nfull : 0;
+    char* const at = bits_space(
+        p, kExchangeCounterBytes + nsplit * sa.nparts * sa.nwl * split_vectors(dp) * 64 * sizeof(f32x4), mb.bytes);
+    if (at) {
+      mb.words = (uint32_t*)at;
+      mb.cls = (unsigned char*)at + mb.words_bytes;
+      const hipError_t err = launch_mask_bits(mb, s);
+      if (err != hipSuccess) return err;
+      const int64_t nblk = (mb.rows + kPipeNw * 32 - 1) / (kPipeNw * 32);
+      p.bits = mb.words;
+      p.bit_cls = mb.cls;
+      p.bit_rows = mb.rows;
+      p.bits_h = mb.heads > 1 ? (int64_t)mb.nt * mb.rows : 0;
+      p.bits_b = mb.batch > 1 ? (int64_t)mb.heads * mb.nt * mb.rows : 0;
+      p.cls_h = mb.heads > 1 ? nblk * mb.nt : 0;
+      p.cls_b = mb.batch > 1 ? mb.heads * nblk * mb.nt : 0;
+      return launch_pipe16_bits(p, sa, dk, bf16, prescale, s);
     }
-    if (bf16)
-      return causal ? launch_narrow<__bf16, true>(p, sa, dk, s) : launch_narrow<__bf16, false>(p, sa, dk, s);
-    return causal ? launch_narrow<_Float16, true>(p, sa, dk, s) : launch_narrow<_Float16, false>(p, sa, dk, s);
   }
-  if (p.mask_kind != MASK_NONE) {  // with causal, a pair must pass both rules
-    if (bf16)
-      return causal ? launch_bucket<__bf16, true, false, 16>(p, sa, dk, s)
-                    : launch_bucket<__bf16, false, false, 16>(p, sa, dk, s);
-    if (prescale)
-      return causal ? launch_bucket<_Float16, true, true, 16>(p, sa, dk, s)
-                    : launch_bucket<_Float16, false, true, 16>(p, sa, dk, s);
-    return causal ? launch_bucket<_Float16, true, false, 16>(p, sa, dk, s)
-                  : launch_bucket<_Float16, false, false, 16>(p, sa, dk, s);
-  }
-  if (bf16)
-    return causal ? launch_bucket<__bf16, true, false>(p, sa, dk, s) : launch_bucket<__bf16, false, false>(p, sa, dk, s);
-  if (prescale)
-    return causal ? launch_bucket<_Float16, true, true>(p, sa, dk, s) : launch_bucket<_Float16, false, true>(p, sa, dk, s);
-  return causal ? launch_bucket<_Float16, true, false>(p, sa, dk, s) : launch_bucket<_Float16, false, false>(p, sa, dk, s);
+  if (dk > 128) return launch_pipe16_wide(p, sa, dk, bf16, causal, prescale, s);
+  return launch_pipe16_kernel(p, sa, dk, bf16, causal, prescale, s);
 }
 
 void describe_pipe16(int dk, int B, int H, int Sq, int Sk, bool causal, bool narrow, char* buf, int len) {

@@ -28,6 +28,7 @@
 // attention_fwd_lse / attention_bwd: the training pair (no reference
 // counterpart: the reference is forward-only, cmpext3/__init__.py:115-125),
 // used by cmpext3's autograd Function.
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -113,8 +114,10 @@ int launch(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& 
   }
   const int B = (int)q.size(0), H = (int)q.size(1), Hkv = (int)k.size(1), Sq = (int)q.size(2),
             Sk = (int)k.size(2);
-  const Workspace ws = workspace_for(
-      q, stream, cmpext3_attn_fwd_workspace_size(dtype, B, H, Hkv, Sq, Sk, D, mask.dtype, causal ? 1 : 0, 0));
+  size_t need = cmpext3_attn_fwd_workspace_size(dtype, B, H, Hkv, Sq, Sk, D, mask.dtype, causal ? 1 : 0, 0);
+  const size_t bits = cmpext3_attn_fwd_mask_workspace_size(dtype, B, H, Hkv, Sq, Sk, D, mask.dtype, ms, causal ? 1 : 0);
+  if (bits > 0) need = std::max(need, (size_t)CMPEXT3_WORKSPACE_COUNTER_BYTES) + bits;
+  const Workspace ws = workspace_for(q, stream, need);
   return cmpext3_attn_fwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dtype, B, H, Hkv, Sq,
                              Sk, D, qs, ks, vs, os, mask.dtype >= 0 ? mask.t.data_ptr() : nullptr,
                              mask.dtype, ms, scale, causal ? 1 : 0, ws.ptr, ws.bytes, stream);
