@@ -952,7 +952,9 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     const int sb = g.sb, ps = g.pstride;
     const int nwl = sa.nwl;  // waves past it hold no rows and left above
     const __amdgpu_buffer_rsrc_t wsr = uniform_rsrc(sa.ws, (int64_t)(sb + 1) * ps * nwl * NV * 64 * 16);
-    auto voff = [&](int q, int k) { return ((((sb * ps + q) * nwl + wave) * NV + k) * 64 + lane) * 16; };
+    // vector k of part q: a scalar offset, the lane's 16 bytes on the vector side
+    auto soff = [&](int q, int k) { return (((sb * ps + q) * nwl + wv) * NV + k) * 1024; };
+    const int l16 = lane * 16;
     // Every lane moves its vectors, also lanes of rows past Sq (a decode
     // step's wave holds one or two live rows): whole 1 KB runs per
     // instruction measured faster than the sparse 16-byte pieces of the live
@@ -961,9 +963,11 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     // device-scope (aux 16 = sc1) 16-byte accesses; the builtins move dwords, so the
     // fp32 values go through explicit bit casts
     auto st_ws = [&](f32x4 x, int off) {
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), wsr, off, 0, 16);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), wsr, l16, off, 16);
     };
-    auto ld_ws = [&](int off) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(wsr, off, 0, 16)); };
+    auto ld_ws = [&](int off) {
+      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(wsr, l16, off, 16));
+    };
     int* const ctr = sa.cnt + 2 * (sb * nwl + wave);  // {parts arrived, states written}
     // a part whose keys are all masked for this row holds nothing: offset -inf
     const float m_own = lsum > 0.f ? mb : -INFINITY;
@@ -973,9 +977,6 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     // not depend on which one writes (reruns stay bit-identical); rounding O/l
     // to fp16 before the merge adds at most one fp16 rounding to the output.
     const bool half_x = std::is_same<T, _Float16>::value && (nparts == 2 || STREAMK);
-    auto ml_off = [&](int q) {
-      return ((((sb * ps + q) * nwl + wave) * NV + 2 * NDB) * 64) * 16 + lane * 8;
-    };
     u32x4 own_h[2 * NDB];  // half_x: this part's O / l in fp16
     if (half_x) {
       const float il = lsum > 0.f ? 1.f / lsum : 0.f;
@@ -989,17 +990,17 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
       if (half_x) {
 #pragma unroll
         for (int v = 0; v < 2 * NDB; ++v)
-          __builtin_amdgcn_raw_buffer_store_b128(own_h[v], wsr, voff(part, v), 0, 16);
+          __builtin_amdgcn_raw_buffer_store_b128(own_h[v], wsr, l16, soff(part, v), 16);
         __builtin_amdgcn_raw_buffer_store_b64((u32x2){__float_as_uint(m_own), __float_as_uint(lsum)}, wsr,
-                                              ml_off(part), 0, 16);
+                                              lane * 8, soff(part, 2 * NDB), 16);
       } else {
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
           for (int g = 0; g < 4; ++g)
             st_ws((f32x4){oacc[db][4 * g], oacc[db][4 * g + 1], oacc[db][4 * g + 2], oacc[db][4 * g + 3]},
-                  voff(part, db * 4 + g));
-        st_ws((f32x4){m_own, lsum, 0.f, 0.f}, voff(part, NDB * 4));
+                  soff(part, db * 4 + g));
+        st_ws((f32x4){m_own, lsum, 0.f, 0.f}, soff(part, NDB * 4));
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
@@ -1037,56 +1038,68 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
       if (lane == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("" ::: "memory");  // the exchange loads stay after the counters
-    // Merge every part in part order, this one from its registers: the same
-    // instructions on the same values whichever part arrives last, so a
-    // rerun is bit-identical.
+    // Merge every part in part order: the same operations on the same values
+    // whichever part arrives last, so a rerun is bit-identical.
     auto ml_of = [&](int q) -> f32x2 {
       if (q == part) return (f32x2){m_own, lsum};
       if (half_x) {
-        const u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wsr, ml_off(q), 0, 16));
+        const u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wsr, lane * 8, soff(q, 2 * NDB), 16));
         return (f32x2){__uint_as_float(w[0]), __uint_as_float(w[1])};
       }
-      const f32x4 x = ld_ws(voff(q, NDB * 4));
+      const f32x4 x = ld_ws(soff(q, NDB * 4));
       return (f32x2){x[0], x[1]};
     };
-    // fp32 exchange: the loads of CH parts are issued together (one memory
-    // round trip per CH parts, not per part); part indices past the last are
-    // clamped to it and dropped, the own part's loads (of whatever its slot
-    // holds) are replaced by its registers.
-    constexpr int CH = 4;                   // parts per batch of offset loads
-    constexpr int CH2 = NDB <= 2 ? 2 : 1;   // parts per batch of O loads (registers)
-    float mt = m_own;
-    if (half_x) {
+    // fp32 exchange.  A part's O comes back in NB batches of BV vectors, one
+    // batch in flight while the one before it is added: the merge is the
+    // launch's tail, and each memory round trip of it shows.  (From D = 128
+    // a whole part does not fit the registers beside the accumulators; asked
+    // for it, the compiler waited for every vector by itself: bf16 D = 256,
+    // two parts of 32 blocks, 42 us for 28 unsplit.)
+    constexpr int NB = NDB > 3 ? 2 : 1, BV = NDB * 4 / NB;
+    auto load = [&](f32x4 (&x)[BV], int q, int b) {
+#pragma unroll
+      for (int v = 0; v < BV; ++v) x[v] = ld_ws(soff(q, b * BV + v));
+    };
+    auto weight = [&](float m) { return m == -INFINITY ? 0.f : fast_exp2(m - moff); };
+    float lnew = 0.f;
+    if (half_x && nparts == 2) {
+      // O / l in fp16, weighted by a * l: the other part's all at once
+      u32x4 x[2 * NDB];
+      const f32x2 mo = ml_of(1 - part);
+#pragma unroll
+      for (int v = 0; v < 2 * NDB; ++v) x[v] = __builtin_amdgcn_raw_buffer_load_b128(wsr, l16, soff(1 - part, v), 16);
+      __builtin_amdgcn_sched_barrier(0);
+      moff = fmaxf(m_own, mo[0]);
+      const bool first = part == 0;
+      const float ao = weight(mo[0]), as = weight(m_own);
+      const float wo = ao * mo[1], ws = as * lsum;
+      lnew = first ? __builtin_fmaf(mo[1], ao, ws) : __builtin_fmaf(lsum, as, wo);
+#pragma unroll
+      for (int v = 0; v < 2 * NDB; ++v)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const f32x2 f = Elt<T>::unpack(x[v][w]), e = Elt<T>::unpack(own_h[v][w]);
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            oacc[v / 2][8 * (v & 1) + 2 * w + u] =
+                first ? __builtin_fmaf(f[u], wo, e[u] * ws) : __builtin_fmaf(e[u], ws, f[u] * wo);
+        }
+    } else if (half_x) {
+      float mt = m_own;
       for (int q = 0; q < nparts; ++q)
         if (q != part) mt = fmaxf(mt, ml_of(q)[0]);
-    } else {
-      for (int q0 = 0; q0 < nparts; q0 += CH) {
-        float mq[CH];
+      moff = mt;
 #pragma unroll
-        for (int j = 0; j < CH; ++j) mq[j] = ld_ws(voff(min(q0 + j, nparts - 1), NDB * 4))[0];
-#pragma unroll
-        for (int j = 0; j < CH; ++j)
-          if (q0 + j < nparts && q0 + j != part) mt = fmaxf(mt, mq[j]);
-      }
-    }
-    moff = mt;
-    f32x16 own[NDB];
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) {
-      own[db] = oacc[db];
-      oacc[db] = (f32x16){};
-    }
-    float lnew = 0.f;
-    if (half_x) {
+      for (int db = 0; db < NDB; ++db) oacc[db] = (f32x16){};
       for (int q = 0; q < nparts; ++q) {  // O / l in fp16, weighted by a * l
         const f32x2 ml = ml_of(q);
-        const float a = ml[0] == -INFINITY ? 0.f : fast_exp2(ml[0] - mt);
+        const float a = weight(ml[0]);
         lnew = __builtin_fmaf(ml[1], a, lnew);
         const float wq = a * ml[1];
 #pragma unroll
         for (int v = 0; v < 2 * NDB; ++v) {
           const u32x4 x = q == part ? own_h[v]
-                                    : __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wsr, voff(q, v), 0, 16));
+                                    : __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wsr, l16, soff(q, v), 16));
 #pragma unroll
           for (int w = 0; w < 4; ++w) {
             const f32x2 f = Elt<T>::unpack(x[w]);
@@ -1096,32 +1109,86 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
           }
         }
       }
+    } else if (nparts == 2) {
+      // the other part's state, joined to this one's registers in part order
+      f32x4 xa[BV], xb[BV];
+      const f32x2 mo = ml_of(1 - part);
+      load(xa, 1 - part, 0);
+      if constexpr (NB == 2) load(xb, 1 - part, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      moff = fmaxf(m_own, mo[0]);
+      const float wo = weight(mo[0]), ws = weight(m_own);
+      const bool first = part == 0;
+      lnew = first ? __builtin_fmaf(mo[1], wo, lsum * ws) : __builtin_fmaf(lsum, ws, mo[1] * wo);
+      auto join = [&](const f32x4 (&x)[BV], int b) {
+#pragma unroll
+        for (int v = 0; v < BV; ++v)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int db = (b * BV + v) / 4, r = 4 * ((b * BV + v) & 3) + i;
+            const float o = oacc[db][r];
+            oacc[db][r] = first ? __builtin_fmaf(x[v][i], wo, o * ws) : __builtin_fmaf(o, ws, x[v][i] * wo);
+          }
+      };
+      join(xa, 0);
+      if constexpr (NB == 2) join(xb, 1);
     } else {
-      for (int q0 = 0; q0 < nparts; q0 += CH2) {
-        f32x4 ml[CH2], x[CH2][NDB * 4];
+      // every part's state from the exchange, this one's too, in part order
+      constexpr int CH = 4;  // parts per batch of offset loads
+      float mt = m_own;
+      for (int q0 = 0; q0 < nparts; q0 += CH) {
+        float mq[CH];
 #pragma unroll
-        for (int j = 0; j < CH2; ++j) {
-          const int qq = min(q0 + j, nparts - 1);
-          ml[j] = ld_ws(voff(qq, NDB * 4));
+        for (int j = 0; j < CH; ++j) mq[j] = ld_ws(soff(min(q0 + j, nparts - 1), NDB * 4))[0];
 #pragma unroll
-          for (int v = 0; v < NDB * 4; ++v) x[j][v] = ld_ws(voff(qq, v));
+        for (int j = 0; j < CH; ++j) mt = fmaxf(mt, mq[j]);
+      }
+      moff = mt;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) oacc[db] = (f32x16){};
+      auto add = [&](const f32x4 (&x)[BV], int b, float w) {
+#pragma unroll
+        for (int v = 0; v < BV; ++v)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int db = (b * BV + v) / 4, r = 4 * ((b * BV + v) & 3) + i;
+            oacc[db][r] = __builtin_fmaf(x[v][i], w, oacc[db][r]);
+          }
+      };
+      f32x4 xa[BV], xb[BV];
+      auto ml_at = [&](int q) { return ld_ws(soff(min(q, nparts - 1), NDB * 4)); };
+      f32x4 ma = ml_at(0);
+      load(xa, 0, 0);
+      if constexpr (NB == 2) {
+        for (int q = 0; q < nparts; ++q) {
+          load(xb, q, 1);
+          __builtin_amdgcn_sched_barrier(0);
+          const float w = weight(ma[0]);
+          lnew = __builtin_fmaf(ma[1], w, lnew);
+          add(xa, 0, w);
+          __builtin_amdgcn_sched_barrier(0);
+          ma = ml_at(q + 1);
+          load(xa, min(q + 1, nparts - 1), 0);
+          __builtin_amdgcn_sched_barrier(0);
+          add(xb, 1, w);
         }
-#pragma unroll
-        for (int j = 0; j < CH2; ++j) {
-          const int q = q0 + j;
-          if (q >= nparts) break;
-          const bool mine = q == part;
-          const float mq = mine ? m_own : ml[j][0];
-          const float a = mq == -INFINITY ? 0.f : fast_exp2(mq - mt);
-          lnew = __builtin_fmaf(mine ? lsum : ml[j][1], a, lnew);
-#pragma unroll
-          for (int db = 0; db < NDB; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                oacc[db][4 * g + i] =
-                    __builtin_fmaf(mine ? own[db][4 * g + i] : x[j][db * 4 + g][i], a, oacc[db][4 * g + i]);
+      } else {
+        for (int q = 0; q < nparts; q += 2) {
+          const f32x4 mb2 = ml_at(q + 1);
+          load(xb, min(q + 1, nparts - 1), 0);
+          __builtin_amdgcn_sched_barrier(0);
+          const float wa = weight(ma[0]);
+          lnew = __builtin_fmaf(ma[1], wa, lnew);
+          add(xa, 0, wa);
+          __builtin_amdgcn_sched_barrier(0);
+          if (q + 1 < nparts) {
+            ma = ml_at(q + 2);
+            load(xa, min(q + 2, nparts - 1), 0);
+            __builtin_amdgcn_sched_barrier(0);
+            const float wb = weight(mb2[0]);
+            lnew = __builtin_fmaf(mb2[1], wb, lnew);
+            add(xb, 0, wb);
+          }
         }
       }
     }
