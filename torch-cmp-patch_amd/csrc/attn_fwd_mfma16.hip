@@ -87,7 +87,7 @@ bool short16_applies(const FwdParams& p, int dk, bool causal);
 hipError_t launch_short16(const FwdParams& p, int dk, bool bf16, hipStream_t s);
 void describe_short16(int dk, int Sq, int Sk, char* buf, int len);
 hipError_t launch_pipe16(const FwdParams& p, int dk, bool bf16, bool causal, bool prescale, hipStream_t s);
-void describe_pipe16(int dk, int B, int H, int Sq, int Sk, bool causal, bool narrow, char* buf, int len);
+void describe_pipe16(int dk, int B, int H, int Sq, int Sk, bool causal, bool narrow, bool bf16, char* buf, int len);
 bool packs_query_heads(const FwdParams& p, bool causal, bool masked_rows);
 void pack_query_heads(FwdParams& p);
 bool decode16_applies(const FwdParams& p, bool causal);
@@ -201,7 +201,7 @@ void describe_mfma16(int D, int B, int H, int Sq, int Sk, bool causal, bool bf16
   // (narrow rows above 128 stay here; the default scale: fp16 pre-scales Q)
   const bool wide = dk > 128;
   if ((!elem || (D % 2 == 0 && !wide)) && pipe16_applies(p, dk) && !(wide && keeps_wide(dk, causal, !bf16))) {
-    describe_pipe16(elem ? (dk <= 64 ? 64 : 128) : dk, B, H, Sq, Sk, causal, elem, buf, len);
+    describe_pipe16(elem ? (dk <= 64 ? 64 : 128) : dk, B, H, Sq, Sk, causal, elem, bf16, buf, len);
     if (elem) snprintf(buf + strlen(buf), len - strlen(buf), " narrow rows");
     return;
   }

@@ -25,6 +25,8 @@ constexpr int kMinPartTiles = 8;
 constexpr int kMaxPartsPerCu = 2;
 constexpr int kMaxCausalParts = 8;       // parts per causal block at most
 constexpr int kMinCausalPartTiles = 16;  // tiles of a causal block's longest part at least
+constexpr int kMinManyCausalTiles = 24;  // the same with more than two parts
+constexpr int kMinTailTiles = 32;        // tiles of a prefill block whose last half round is cut
 constexpr int kLongCausalTiles = 64;     // a long causal sweep (the last block's tiles)
 constexpr int kMi355xCus = 256;  // used when no device is visible (host-only calls)
 
@@ -80,6 +82,50 @@ int exchange_waves(int n_qblk, int Sq) {
   return n_qblk > 1 ? kPipeNw : (Sq + 31) / 32 < kPipeNw ? (Sq + 31) / 32 : kPipeNw;
 }
 
+// What the plan weighs besides the grid: the head-dim bucket, whether two
+// parts exchange O in 16 bits (fp16), and whether the block is short (decode,
+// packed rows: at most 64 rows, a launch bound by the K/V stream).
+struct PlanKind {
+  int dk;
+  bool half, shortq;
+};
+
+// Cost of cutting a block's sweep in two, in key tiles of one block: the
+// prologue, the exchange and the merge of one block (about 3 us) and each
+// further block's share of the exchange's bytes.  Fitted on MI355X to
+// [1,H,S,S,D] with 32 to 240 blocks (D = 48, 64, 128 and 256, S = 512 to
+// 3072): where it exceeds the tiles a cut saves, the cut launch was the slower
+// one, by up to half (bf16 [1,32,1024,1024,128], 256 blocks: 24 us whole, 37
+// us cut), and with few exceptions only there.
+float cut_cost(const PlanKind& k, int n) {
+  const float per_block = k.dk > 128 ? 0.057f : k.dk > 64 ? (k.half ? 0.063f : 0.114f) : (k.half ? 0.034f : 0.063f);
+  const float base = !k.half || k.dk > 128 ? 6.f : k.dk > 64 ? 7.f : 8.f;
+  return base + per_block * n;
+}
+
+// Parts of every block of a non-causal prefill with fewer blocks than CUs.
+// With a part to a CU, P parts save nt (1 - 1/P) tiles; two parts beyond that
+// share CUs and save 0.38 nt (above D = 128 a CU holds one workgroup: nothing).  Three parts and more all leave fp32 states, and
+// from four on a launch pays another 5 (D > 128) or 12 tiles: bf16
+// [1,8,1024,1024,D], 64 blocks, whole / in 2 / 3 / 4 parts, D = 64: 16.1 / 13.8
+// / 12.8 / 17.2 us, D = 128: 21.5 / 19.9 / 19.4 / 23.1, D = 256: 46.7 / 37.5 /
+// 34.3 / 37.1.
+int prefill_parts(const PlanKind& k, int n, int nt, int cus, int occ) {
+  const float save2 = nt * (2 * n <= cus ? 0.5f : occ > 1 ? 0.38f : 0.f) - cut_cost(k, n);
+  int parts = save2 > 0.f ? 2 : 1;
+  float best = save2 > 0.f ? save2 : 0.f;
+  const PlanKind full = {k.dk, false, false};
+  for (int p = 3; p <= nt / kMinPartTiles && n * p <= cus; ++p) {
+    const float many = p > 3 ? (k.dk > 128 ? 5.f : 12.f) : k.dk > 64 && k.dk <= 128 ? 2.f : 0.f;
+    const float save = nt * (1.f - 1.f / p) - cut_cost(full, n * p / 2) - many;
+    if (save > best) {
+      best = save;
+      parts = p;
+    }
+  }
+  return parts;
+}
+
 // Which blocks run whole and how the rest are cut.  n blocks on `cus` CUs at
 // `occ` workgroups per CU; the dispatcher hands workgroup i to CU i mod cus
 // while all of them fit, so after the whole rounds each CU takes exactly one
@@ -94,13 +140,17 @@ int exchange_waves(int n_qblk, int Sq) {
 // parts so that one round holds them all, the longest part keeping at least
 // kMinCausalPartTiles tiles: each block's longest part, and so the launch,
 // gets shorter.  Measured on MI355X (same run): [1,4,8192,128] bf16 135 ->
-// 98 us, [1,8,2048,256] 85 -> 73 us, [1,16,2048,64] fp16 30 -> 25 us,
-// [1,8,1024,64] 17 -> 14 us; shorter sweeps on busy CUs lost to the parts'
+// 98 us, [1,8,2048,256] 85 -> 54 us, [1,8,1024,64] 17.2 -> 13.8 us; shorter
+// sweeps on busy CUs lost to the parts'
 // prologues and merges ([1,32,1024,128] 25 -> 28 us, [1,32,512,128] 16 ->
-// 18 us) and stay whole.  Every part of every block keeps at least one tile
+// 18 us) and stay whole.  More than two parts want longer ones
+// (kMinManyCausalTiles: bf16 [1,16,2048,64] 29.2 whole, 23.1 in 2, 26.7 in 3;
+// [1,8,2048,128] 39.2 / 27.1 / 27.9, 35.3 in 4), and beyond the smallest
+// grids more than three lose ([1,8,3072,64] 25.3 in 3, 32.1 in 4).  Every part
+// of every block keeps at least one tile
 // (a causal row sees a key in the first tile of a part, or none of the part's
 // keys: its state then has no weight in the merge).
-SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntiles_min) {
+SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntiles_min, const PlanKind& k) {
   SplitArgs sa = {n, 1, nullptr, nullptr, kPipeNw};
   if (cus <= 0) return sa;
   if (causal) {
@@ -108,6 +158,9 @@ SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntile
     if (n * 2 > slots || (n * 2 > cus && ntiles < kLongCausalTiles)) return sa;
     int parts = slots / n;
     if (parts > ntiles / kMinCausalPartTiles) parts = ntiles / kMinCausalPartTiles;
+    if (parts > 2 && parts > ntiles / kMinManyCausalTiles)
+      parts = ntiles / kMinManyCausalTiles > 2 ? ntiles / kMinManyCausalTiles : 2;
+    if (parts > 3 && n * 3 > cus) parts = 3;
     if (parts > ntiles_min) parts = ntiles_min;
     if (parts > kMaxCausalParts) parts = kMaxCausalParts;
     if (parts < 2) return sa;
@@ -117,13 +170,27 @@ SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntile
   }
   const int full = n / cus, rem = n - full * cus;
   if (rem == 0 || full + 1 > occ) return sa;  // whole rounds, or more than fits at once
-  // After whole rounds each CU takes one part of the round that remains.  With
-  // no whole round (fewer blocks than CUs: decode, short sweeps) each CU can
-  // hold several parts at once: more key ranges streamed side by side, more
-  // loads in flight (a decode step with one part per CU reaches ~5.2 TB/s).
-  const int per_cu = full == 0 ? (occ < kMaxPartsPerCu ? occ : kMaxPartsPerCu) : 1;
-  int parts = per_cu * cus / rem;
-  if (parts > ntiles / kMinPartTiles) parts = ntiles / kMinPartTiles;
+  int parts;
+  if (full == 0 && !k.shortq) {
+    parts = prefill_parts(k, n, ntiles, cus, occ);
+  } else {
+    // After whole rounds each CU takes at most one part of the round that
+    // remains.  With no whole round of short blocks (decode, short sweeps) each
+    // CU can hold several parts at once: more key ranges streamed side by side,
+    // more loads in flight (a decode step with one part per CU reaches ~5.2
+    // TB/s).
+    const int per_cu = full == 0 ? (occ < kMaxPartsPerCu ? occ : kMaxPartsPerCu) : 1;
+    parts = per_cu * cus / rem;
+    if (parts > ntiles / kMinPartTiles) parts = ntiles / kMinPartTiles;
+    if (full > 0 && !k.shortq) {
+      // the tail of a prefill: two parts (bf16 [1,20,2048,2048,64], 64 blocks
+      // left: whole 35.8 us, 2 parts 31.8, 3 32.2, 4 33.9), and where each CU
+      // would take little less than a whole block more, only of long sweeps
+      // ([1,64,768,768,64], 128 left: 17.9 whole, 18.2 cut; 1536: 29.8, 28.1)
+      if (parts > 2) parts = 2;
+      if (rem * 2 >= cus && ntiles < kMinTailTiles) parts = 1;
+    }
+  }
   if (parts < 2) return sa;
   sa.nfull = full * cus;
   sa.nparts = parts;
@@ -140,23 +207,28 @@ SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntile
 // merges than they balance; the counters take 2 per (block, wave).
 constexpr int kMaxStreamkWaves = kExchangeCounters / 2;
 
-bool streamk_applies(const FwdParams& p, int n, int dk, int occ, int cus, bool causal) {
+bool streamk_applies(const FwdParams& p, int n, int dk, int occ, int cus, bool causal, bool half) {
   if (causal || p.lse || p.elem_rows || p.mask_kind != MASK_NONE || p.pack_sq > 0) return false;
   if (!(dk == 32 || dk == 64 || dk == 128) || p.Sq <= (kPipeNw - 2) * 32) return false;
   const int slots = occ * cus;
   if (cus <= 0 || n < cus || n % slots == 0 || n * kPipeNw > kMaxStreamkWaves) return false;
-  // Only where the classic plan leaves slots idle for the whole launch: one
-  // partial round of whole CUs (n a multiple of the CU count: no block left
-  // to split), or, at two workgroups per CU, a last round at most half full.
-  // Where the classic plan splits the blocks past the whole CUs, it measured
-  // faster (SDXL self-attention 91.1 us against 97.7 us stream-K, same run:
-  // every stream-K share pays a second prologue and every block a merge);
-  // [2,4,4096,4096,64], one block per CU, 54.6 us unsplit against 44.8 us.
-  const bool idle_round = n < slots && n % cus == 0;
-  const bool thin_tail = n > slots && occ == 2 && n % slots <= slots / 2;
+  // Only where the classic plan leaves slots idle for the whole launch and the
+  // sweeps are long enough to repay a second prologue per share and a merge
+  // per block: one block per CU (no block left to split; D <= 64 fp16
+  // [2,4,4096,4096,64] 48.9 -> 44.5 us, bf16 50.7 -> 46.7, but 28.1 -> 31.6 at
+  // 2048 keys; D = 128 fp16 77.3 -> 74.0, bf16 72.9 -> 74.7), or, at two
+  // workgroups per CU, a last round at most a quarter full (bf16
+  // [2,10,4096,4096,128], 640 blocks, 187 -> 180; half full, 768 blocks of
+  // [1,32,3072,3072,128], 153 -> 160).  Two blocks per CU of three lose on
+  // shorter sweeps ([1,32,2048,2048,64] 41.4 -> 46.7).  Where the classic plan splits the
+  // blocks past the whole CUs, it measured faster (SDXL self-attention 91.1 us
+  // against 97.7 us stream-K, same run).
+  const int nt = n_key_tiles(p.Sk);
+  const bool idle_round = n < slots && n % cus == 0 && (dk > 64 ? half && nt >= 128 : nt >= (n == cus ? 72 : 128));
+  const bool thin_tail = n > slots && occ == 2 && n % slots <= slots / 4 && nt >= 64;
   if (!idle_round && !thin_tail) return false;
   const int64_t rounds = (n + slots - 1) / slots;
-  return (int64_t)n * n_key_tiles(p.Sk) / (rounds * slots) >= kMinPartTiles;
+  return (int64_t)n * nt / (rounds * slots) >= kMinPartTiles;
 }
 
 // The stream-K launch: workgroup count and part slots per block (an upper
@@ -332,7 +404,7 @@ hipError_t launch_pipe16(const FwdParams& p0, int dk0, bool bf16, bool causal, b
   const int dp = (dk + 31) / 32 * 32;
   // stream-K where it applies and its exchange fits the space this call has
   size_t sk_need = 0;
-  if (streamk_applies(p, n, dk, occ, cus, causal)) {
+  if (streamk_applies(p, n, dk, occ, cus, causal, !bf16)) {
     SplitArgs sk = streamk_plan(n, n_key_tiles(p.Sk), occ, cus);
     const size_t part_bytes = (size_t)n * kPipeNw * split_vectors(dp) * 64 * sizeof(f32x4);
     const int fit = bind_exchange(p, sk.nparts, part_bytes, 2 * n * kPipeNw, &sk.ws, &sk.cnt);
@@ -343,7 +415,8 @@ hipError_t launch_pipe16(const FwdParams& p0, int dk0, bool bf16, bool causal, b
     }
   }
   const int n_qblk = (p.Sq + kPipeNw * 32 - 1) / (kPipeNw * 32);
-  SplitArgs sa = split_plan(n, causal_tiles(p.Sk, n_qblk, causal), occ, cus, causal, causal_tiles(p.Sk, 1, causal));
+  SplitArgs sa = split_plan(n, causal_tiles(p.Sk, n_qblk, causal), occ, cus, causal, causal_tiles(p.Sk, 1, causal),
+                            {dk, !bf16, p.Sq <= (kPipeNw - 2) * 32});
   sa.nwl = exchange_waves((p.Sq + kPipeNw * 32 - 1) / (kPipeNw * 32), p.Sq);
   if (p.dry) *p.dry = SplitInfo{0, 1};  // the stream-K attempt's record, if any, is not this plan
   if (sa.nparts > 1) {
@@ -387,19 +460,19 @@ hipError_t launch_pipe16(const FwdParams& p0, int dk0, bool bf16, bool causal, b
   return launch_pipe16_kernel(p, sa, dk, bf16, causal, prescale, s);
 }
 
-void describe_pipe16(int dk, int B, int H, int Sq, int Sk, bool causal, bool narrow, char* buf, int len) {
+void describe_pipe16(int dk, int B, int H, int Sq, int Sk, bool causal, bool narrow, bool bf16, char* buf, int len) {
   const int bq = kPipeNw * 32;
   const int n = n_blocks(B, H, Sq);
   const int n_qblk = (Sq + bq - 1) / bq;
   const SplitArgs sa = split_plan(n, causal_tiles(Sk, n_qblk, causal), pipe_occ(dk), device_cus(), causal,
-                                  causal_tiles(Sk, 1, causal));
+                                  causal_tiles(Sk, 1, causal), {dk, !bf16, Sq <= (kPipeNw - 2) * 32});
   char split[96] = "";
   FwdParams p = {};
   p.Sq = Sq;
   p.Sk = Sk;
   p.mask_kind = MASK_NONE;
   p.elem_rows = narrow ? 4 : 0;
-  if (streamk_applies(p, n, dk, pipe_occ(dk), device_cus(), causal)) {
+  if (streamk_applies(p, n, dk, pipe_occ(dk), device_cus(), causal, !bf16)) {
     const SplitArgs sk = streamk_plan(n, n_key_tiles(Sk), pipe_occ(dk), device_cus());
     snprintf(split, sizeof split, " stream-K: %d workgroups x %lld tiles of %d blocks (with a workspace)", sk.sk_wgs,
              (long long)n * n_key_tiles(Sk) / sk.sk_wgs, n);
