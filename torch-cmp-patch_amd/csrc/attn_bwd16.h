@@ -80,22 +80,59 @@ struct BwdParams {
   int nfull, nfull_q;
 };
 
+// Time of a gradient sweep cut into ns parts per block, in us: `tiles` tiles of
+// tile_us each in the longest block, n_wg blocks, and beyond one part the
+// launch that adds the fp32 partials and their way to memory and back (part_mb
+// MB per part of all blocks).  Workgroups sharing a CU slow each other: two
+// take 1.5 to 1.6 times as long as one, three twice (one per CU above D = 128:
+// rounds).  A causal launch does half the work; while its workgroups are all
+// resident the longest sets its time.  Least squares over 371 backward calls on
+// MI355X (8 to 64 heads, 100 to 3072 tokens, f16/bf16 D = 64, 128, 256 and fp32
+// D = 40, 64, 128, each whole and in up to two plans).
+inline float sweep_us(int64_t n_wg, int ns, int occ, int cus, bool causal, int64_t tiles, float tile_us,
+                      float part_mb) {
+  float k = (float)(n_wg * ns) / cus;
+  if (!causal) k = __builtin_ceilf(k);
+  const float step = occ == 2 ? 0.63f : 0.52f, full = 1.f + step * (occ - 1);
+  float h = k <= 1.f ? 1.f : k <= occ ? 1.f + step * (k - 1.f) : full * k / occ;
+  if (causal && k > 1.f) {
+    const float resident = 1.f + 0.1f * step * ((k < occ ? k : occ) - 1.f);
+    const float rounds = 0.5f * h + (occ == 1 ? 0.3f : -0.2f);
+    h = k <= occ || resident > rounds ? resident : rounds;
+  }
+  const float mb = part_mb * ns;
+  const float sum = 2.5f + (mb < 4.f ? 0.375f * mb : 1.5f) + 0.27f * mb + 0.0005f * mb * mb;
+  return tile_us * tiles / ns * h + (ns > 1 ? sum : 0.f);
+}
+
 // Parts per block of a gradient sweep (1 = unsplit).  With too few blocks
 // (n_wg) for the CU slots the kernel's occupancy allows (one 4-wave workgroup
 // per wave per SIMD), each block's sweep is cut into contiguous parts whose
-// fp32 partials are summed afterwards: non-causal, as many parts as fill one
-// round of slots; causal, enough for two rounds, so that longest-first
-// dispatch pairs long parts with short ones (causal sweeps' lengths run from
-// one tile to all of them).  At most 8 parts, each at least 4 tiles of the
-// longest sweep (`tiles`).
-inline int split_sweep(int64_t n_wg, int occ, int cus, bool causal, int64_t tiles) {
+// fp32 partials are summed afterwards.  At most as many as fill one round of
+// slots, causal two (longest-first dispatch then pairs long parts with short
+// ones: causal sweeps' lengths run from one tile to all of them), at most 8,
+// each at least 4 tiles of the longest sweep; fewer, or none, where that is
+// faster by more than 8%: short sweeps of many heads pay more for the partials
+// than they save (bf16 causal [4,16,512,512,128], 256 blocks: 58 us whole,
+// 111 in 4 parts; [4,16,1024,1024,64] 64 whole, 95 in 2).
+inline int split_sweep(int64_t n_wg, int occ, int cus, bool causal, int64_t tiles, float tile_us, float part_mb) {
   const int64_t slots = (int64_t)cus * occ;
   const int64_t want = causal ? 2 * slots : slots;
   if (n_wg <= 0 || n_wg * 2 > want) return 1;
-  int64_t ns = causal ? (want + n_wg - 1) / n_wg : want / n_wg;
-  if (ns > 8) ns = 8;
-  if (ns > tiles / 4) ns = tiles / 4;
-  return ns >= 2 ? (int)ns : 1;
+  int64_t most = causal ? (want + n_wg - 1) / n_wg : want / n_wg;
+  if (most > 8) most = 8;
+  if (most > tiles / 4) most = tiles / 4;
+  if (most < 2) return 1;
+  int ns = (int)most;
+  float best = 0.92f * sweep_us(n_wg, ns, occ, cus, causal, tiles, tile_us, part_mb);
+  for (int i = 1; i < most; ++i) {
+    const float us = sweep_us(n_wg, i, occ, cus, causal, tiles, tile_us, part_mb);
+    if (us < best) {
+      best = us;
+      ns = i;
+    }
+  }
+  return ns;
 }
 
 // Split plan of a backward launch and its workspace: the dK/dV partials

@@ -78,8 +78,11 @@ BwdSplit bwd16_split(int B, int H, int Hkv, int Sq, int Sk, int D, bool causal, 
   const int occ_q = dk <= 64 ? (masked ? 2 : 3) : dk <= 128 ? (masked && causal ? 1 : 2) : 1;
   const int64_t n_kv = (int64_t)B * Hkv * ((Sk + 127) / 128), n_q = (int64_t)B * H * ((Sq + 127) / 128);
   const int64_t t_kv = (int64_t)(H / Hkv) * ((Sq + 31) / 32), t_q = (Sk + 31) / 32;
-  sp.ns_kv = split_sweep(n_kv, occ_kv, cus, causal, t_kv);
-  sp.ns_q = split_sweep(n_q, occ_q, cus, causal, t_q);
+  // us per 32-row tile of one block, a CU to itself
+  const float us_kv = dk <= 64 ? 0.74f : dk <= 128 ? 1.2f : dk <= 192 ? 2.f : 2.8f;
+  const float us_q = dk <= 64 ? 0.49f : dk <= 128 ? 0.86f : dk <= 192 ? 1.35f : 1.83f;
+  sp.ns_kv = split_sweep(n_kv, occ_kv, cus, causal, t_kv, us_kv, 8e-6f * B * Hkv * Sk * D);
+  sp.ns_q = split_sweep(n_q, occ_q, cus, causal, t_q, us_q, 4e-6f * B * H * Sq * D);
   // non-causal grids past one round: split only the last, partial round
   if (!causal && sp.ns_kv == 1) sp.ns_kv = split_tail(n_kv, occ_kv, cus, t_kv, &sp.nfull_kv);
   if (!causal && sp.ns_q == 1) sp.ns_q = split_tail(n_q, occ_q, cus, t_q, &sp.nfull_q);

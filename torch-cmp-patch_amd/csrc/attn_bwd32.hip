@@ -559,9 +559,14 @@ BwdSplit bwd32_split(int B, int H, int Hkv, int Sq, int Sk, int D, bool causal, 
   if (dk < 0 || (int64_t)B * H * Sq == 0 || Hkv < 1) return sp;
   const int occ_kv = dk <= 32 ? 5 : dk <= 40 ? 4 : dk <= 64 ? (causal ? 4 : 3) : dk <= 128 ? 2 : 1;
   const int occ_q = dk <= 32 ? 7 : dk <= 40 ? 5 : dk <= 64 ? 4 : dk <= 96 ? 3 : dk <= 128 ? 2 : 1;
+  // us per 32-row tile of one block, a CU to itself: about in proportion to the
+  // head dim, 2.2 at D = 40 and 5.0 at 128 for dK/dV; dQ's part that the split
+  // shortens is 0.9, 0.95 and 2.4 at D = 40, 64 and 128
+  const float us_kv = 0.9f + 0.032f * dk, us_q = dk <= 64 ? 0.8f + 0.0024f * dk : 0.019f * dk;
   sp.ns_kv = split_sweep((int64_t)B * Hkv * ((Sk + 63) / 64), occ_kv, cus, causal,
-                         (int64_t)(H / Hkv) * ((Sq + 31) / 32));
-  sp.ns_q = split_sweep((int64_t)B * H * ((Sq + 63) / 64), occ_q, cus, causal, (Sk + 31) / 32);
+                         (int64_t)(H / Hkv) * ((Sq + 31) / 32), us_kv, 8e-6f * B * Hkv * Sk * D);
+  sp.ns_q = split_sweep((int64_t)B * H * ((Sq + 63) / 64), occ_q, cus, causal, (Sk + 31) / 32, us_q,
+                        4e-6f * B * H * Sq * D);
   return sp;
 }
 
