@@ -6,8 +6,8 @@
 // P = softmax(S), S = scale * Q K^T (causal: top-left, key j visible to
 // query i iff j <= i):
 //   Delta_i = sum_d dO_id O_id                     (attn_bwd_delta)
-//   dV = P^T dO,  dK = scale * dS^T Q              (attn_bwd_dkdv, per key block)
-//   dQ = scale * dS K                              (attn_bwd_dq, per query block)
+//   dV = P^T dO,  dK = scale * dS^T Q              (per key block)
+//   dQ = scale * dS K                              (per query block)
 //   with dP = dO V^T and dS = P * (dP - Delta).
 // P is recomputed from the scores and the saved log-sum-exp, so nothing of
 // size Sq x Sk is stored.  The two gradient kernels each own their output rows
@@ -56,11 +56,11 @@ struct BwdParams {
   int B, H, Sq, Sk, D;
   int Hkv;          // K/V heads (dk, dv have Hkv heads); query head h uses K/V head h / group
   int group;        // H / Hkv
-  int n_blk;        // key blocks (dK/dV, per K/V head) or query blocks (dQ, per query head)
-  int n_wg;         // workgroups launched = B * H * n_blk (dK/dV: times nsplit)
+  int n_blk;        // key blocks (dK/dV, per K/V head)
+  int n_blk_q;      // query blocks (dQ, per query head)
+  int n_wg, n_wg_q; // workgroups of the two sweeps
   float c;          // |scale| * log2(e)
   float scale;      // signed scale: dK = scale * dS^T Q, dQ = scale * dS K
-  uint32_t sign;    // 0x80008000 when scale < 0 (XORed into K or Q words), else 0
   // optional attention mask, as in FwdParams (element strides over {batch,
   // head, query}, unit key stride, kind MASK_*; MASK_NONE = none)
   const void* mask;
@@ -78,6 +78,10 @@ struct BwdParams {
   // partials are block-indexed: [nsplit][blocks - nfull][128][D] (likewise
   // nfull_q for dQ)
   int nfull, nfull_q;
+  // 0x80008000 when scale < 0 (XORed into K or Q words), else 0.  Last: from
+  // the middle the compiler widens its load for the vector XOR over the members
+  // beside it, and those stay in scratch
+  uint32_t sign;
 };
 
 // Time of a gradient sweep cut into ns parts per block, in us: `tiles` tiles of
@@ -96,7 +100,7 @@ inline float sweep_us(int64_t n_wg, int ns, int occ, int cus, bool causal, int64
   const float step = occ == 2 ? 0.63f : 0.52f, full = 1.f + step * (occ - 1);
   float h = k <= 1.f ? 1.f : k <= occ ? 1.f + step * (k - 1.f) : full * k / occ;
   if (causal && k > 1.f) {
-    const float resident = 1.f + 0.1f * step * ((k < occ ? k : occ) - 1.f);
+    const float resident = 1.f + (occ > 3 ? 0.18f : 0.1f) * step * ((k < occ ? k : occ) - 1.f);
     const float rounds = 0.5f * h + (occ == 1 ? 0.3f : -0.2f);
     h = k <= occ || resident > rounds ? resident : rounds;
   }
@@ -173,6 +177,18 @@ inline int split_tail(int64_t n, int occ, int cus, int64_t tiles, int* nfull) {
   return (int)ns;
 }
 
+// Whether a dK/dV grid of n blocks leaves (almost) none of its last
+// round of `slots` empty.  Where the dQ sweep runs a wave per SIMD more by itself
+// than beside the dK/dV sweep, such a grid takes its own launch: there is no
+// tail for the dQ workgroups to fill (same MI355X run, in one launch and in two:
+// bf16 causal with a key mask [4,16/8,2048,2048,64] 208 and 199 us; fp32
+// [2,8,3000,3000,40] 812 and 775, causal [2,8,3000,3000,32] 343 and 326; kernels
+// without that wave gain up to 8% from one launch there too, as at bf16 causal
+// [4,16/8,1024,1024,256] 249 and 270).
+inline bool last_round_full(int64_t n, int64_t slots) {
+  return n >= slots && (n + slots - 1) / slots * slots - n <= slots / 10;
+}
+
 // fp32 partial rows of a split sweep ([ns][rows][D], rows = B x heads x S)
 // and where their sum goes: T rows with element strides {batch, head, seq},
 // times `mul`.
@@ -245,25 +261,34 @@ struct TileLoader {
   static constexpr int KCH = DK / 8;
   static constexpr int N = 32 * KCH / 256;  // chunks per thread
   static_assert(32 * KCH % 256 == 0, "whole chunks per thread");
-  int voff[N], loff[N];
-  bool zero[N];
+  // Whole rows per pass of the workgroup (the next chunk's row rides in the
+  // load's scalar offset), or, where a pass is no whole number of rows (DK =
+  // 192), 64-column strips: either way one address register, one LDS offset.
+  // With one of each per chunk the dK/dV sweep at DK = 128 spilled some of them
+  // and waited for the whole fetch to reload them.
+  static constexpr bool BYROW = 256 % KCH == 0;
+  static constexpr int RPP = BYROW ? 256 / KCH : 0;  // rows a pass
+  int voff, loff, step, room;
   __device__ __forceinline__ void init(int tid, int64_t row_stride, int D, int RS) {
-#pragma unroll
-    for (int it = 0; it < N; ++it) {
-      const int ci = it * 256 + tid, r = ci / KCH, c8 = ci - r * KCH;
-      voff[it] = (int)(r * row_stride * 2) + 16 * c8;
-      loff[it] = r * RS + 8 * c8;
-      zero[it] = 8 * c8 >= D;
-    }
+    constexpr int W = BYROW ? KCH : 8;
+    const int r = tid / W, c8 = tid - r * W;
+    voff = (int)(r * row_stride * 2) + 16 * c8;
+    loff = r * RS + 8 * c8;
+    step = (int)(RPP * row_stride * 2);
+    room = D - 8 * c8;  // columns left from this thread's first chunk on
   }
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int soff, u32x4 (&x)[N]) const {
 #pragma unroll
     for (int it = 0; it < N; ++it)
-      x[it] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[it], soff, 0));
+      x[it] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, BYROW ? voff : voff + 128 * it, soff + it * step, 0));
   }
+  template <int RS>
   __device__ __forceinline__ void store(uint16_t* dst, const u32x4 (&x)[N]) const {
 #pragma unroll
-    for (int it = 0; it < N; ++it) *(u32x4*)(dst + loff[it]) = zero[it] ? (u32x4){0u, 0u, 0u, 0u} : x[it];
+    for (int it = 0; it < N; ++it)
+      *(u32x4*)(dst + loff + it * (BYROW ? RPP * RS : 64)) =
+          room <= (BYROW ? 0 : 64 * it) ? (u32x4){0u, 0u, 0u, 0u} : x[it];
   }
 };
 
@@ -317,19 +342,15 @@ __device__ __forceinline__ void store_rows_f32(float* base, int row, int nrows, 
 // ---- dK, dV for one block of 128 keys (4 waves x 32 keys), sweeping the
 // query tiles (32 rows of Q, dO, lse, Delta) through double-buffered LDS.
 // Waves per SIMD: D <= 64: 3 (masked with V parked in LDS; 4 spilled
-// registers), 2 causal; D <= 128: 2 with V parked in LDS (the causal and the
-// masked variants spill 8 registers and are still 12-20% faster than at 1),
+// registers, with two K operands there too), 2 causal; D <= 128: 2 with V parked
+// in LDS (12-20% faster than at 1), the causal and the masked variants with two K operands there too,
 // 1 masked causal (its K/V operands and dK/dV accumulators alone take 192
 // registers); D > 128: 1, with V parked in LDS.
-template <typename T, int DK, bool CAUSAL, bool MASK>
-__global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(DK <= 64 ? (CAUSAL ? 2 : 3) : (DK > 128 || (MASK && CAUSAL)) ? 1 : 2)))
-attn_bwd_dkdv(const BwdParams p) {
-  constexpr int BQ = 32, BKV = 128;
-  constexpr int RS = bwd_lds_stride(DK);  // LDS row stride (halves)
-  constexpr int NKS = DK / 16, NDB = DK / 32;
-  static_assert(DK % 32 == 0, "head-dim bucket");
-  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 2 * BQ * RS];  // [slot][Q, dO][row][col]
+template <int DK, bool CAUSAL, bool MASK>
+struct BwdDkdv {
+  static constexpr int BQ = 32, BKV = 128;
+  static constexpr int RS = bwd_lds_stride(DK);  // LDS row stride (halves)
+  static constexpr int OCC = DK <= 64 ? (CAUSAL ? 2 : 3) : (DK > 128 || (MASK && CAUSAL)) ? 1 : 2;
   // The V operands live in LDS instead of registers where that buys a wave
   // per SIMD: D > 64 (32 fewer VGPRs, two waves instead of one; dK/dV
   // 349 -> 268 us on bf16 [4,16,2048,128], 275 -> 241 us causal, masked
@@ -340,12 +361,35 @@ attn_bwd_dkdv(const BwdParams p) {
   // or causal D <= 64 (three waves with V parked measured slower: 301 -> 327
   // us).  Above D = 128 always: the K operands (DK / 4 registers) and the
   // two accumulators (2 * DK) leave little of one wave's 512 registers.
-  constexpr bool VLDS = DK > 128 ? true : DK > 64 ? !(MASK && CAUSAL) : (MASK && !CAUSAL);
-  constexpr int RSV = DK + 8;
-  __shared__ __attribute__((aligned(16))) uint16_t vpark[VLDS ? BKV * RSV : 8];
+  static constexpr bool VLDS = DK > 128 ? true : DK > 64 ? !(MASK && CAUSAL) : (MASK && !CAUSAL);
+  static constexpr int TILES = 2 * 2 * BQ * RS;           // halves: [slot][Q, dO][row][col]
+  // K operands parked beside V: as many as the registers fall short by.  (A
+  // spilled one is read back inside the tile, behind the next tile's loads:
+  // each tile then waits for memory.  bf16 causal backward with 7 spilled and with
+  // none: [4,16/8,2048,2048,128] 347 -> 329 us, [2,10,4096,4096,128] 380 -> 334;
+  // masked D = 64 with a mask per row [2,10,4096,4096] 1218 -> 930.)
+  static constexpr int KP = DK == 64    ? (MASK && !CAUSAL ? 2 : 0)
+                            : DK == 128 ? (MASK != CAUSAL ? 2 : 0)
+                            : DK == 256 ? (MASK && CAUSAL ? 3 : 0)
+                                        : 0;
+  // halves: an operand is 16 bytes per thread, at consecutive addresses (no
+  // bank conflicts, no padding)
+  static constexpr int PARK = ((VLDS ? DK / 16 : 0) + KP) * 256 * 8 + (VLDS || KP > 0 ? 0 : 8);
   // [slot][-lse2 / c, -Delta][row]: the starting values of the S and dP
   // accumulators, so that the MFMAs leave S - lse2 / c and dP - Delta
-  __shared__ __attribute__((aligned(16))) float lsd[2][2][BQ];
+  static constexpr int LSD = 2 * 2 * BQ;                  // floats
+};
+
+// Workgroup `wg` of the dK/dV sweeps; its LDS arrays (BwdDkdv's sizes).
+template <typename T, int DK, bool CAUSAL, bool MASK>
+__device__ __forceinline__ void bwd_dkdv_block(const BwdParams& p, const int wg, uint16_t* const lds,
+                                               uint16_t* const vpark, float* const lsdp) {
+  using Cfg = BwdDkdv<DK, CAUSAL, MASK>;
+  constexpr int BQ = Cfg::BQ, BKV = Cfg::BKV, RS = Cfg::RS, KP = Cfg::KP;
+  constexpr bool VLDS = Cfg::VLDS;
+  constexpr int NKS = DK / 16, NDB = DK / 32;
+  static_assert(DK % 32 == 0, "head-dim bucket");
+  float (*const lsd)[2][BQ] = (float (*)[2][BQ])lsdp;
 
   const int tid = thread_x(), wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   // (batch, K/V head) and key block; split sweeps: (block, part) pairs as
@@ -357,7 +401,7 @@ attn_bwd_dkdv(const BwdParams p) {
   if (!CAUSAL && p.nfull > 0) {
     // split tail: the first nfull workgroups take whole blocks, the rest
     // ns-way parts of the remaining blocks
-    const int w = block_x();
+    const int w = wg;
     int tile = w;
     part = 0;
     if (w >= p.nfull) {
@@ -374,7 +418,7 @@ attn_bwd_dkdv(const BwdParams p) {
     kb = __builtin_amdgcn_readfirstlane(kb0);
   } else {
     int bh0, vb;
-    kv_tile(block_x(), p.B * p.Hkv, p.n_blk * ns, CAUSAL, bh0, vb);
+    kv_tile(wg, p.B * p.Hkv, p.n_blk * ns, CAUSAL, bh0, vb);
     bhk = __builtin_amdgcn_readfirstlane(bh0);
     vb = __builtin_amdgcn_readfirstlane(vb);
     kb = __builtin_amdgcn_readfirstlane(vb / ns);
@@ -388,8 +432,9 @@ attn_bwd_dkdv(const BwdParams p) {
   // B operands held for the whole sweep: 8 head-dim values of this lane's key
   const uint16_t* kg = (const uint16_t*)p.k + b * p.k_b + hk * p.k_h;
   const uint16_t* vg = (const uint16_t*)p.v + b * p.v_b + hk * p.v_h;
-  u32x4 kf[NKS], vf[VLDS ? 1 : NKS];
-  uint16_t* const vrow = vpark + (wave * 32 + l32) * RSV + 8 * hh;  // this lane's parked V
+  u32x4 kf[NKS - KP], vf[VLDS ? 1 : NKS];
+  u32x4* const vp = (u32x4*)vpark + tid;                // this thread's parked V operands
+  u32x4* const kp = vp + (VLDS ? NKS * 256 : 0);        // and the last KP of K
 #pragma unroll
   for (int s = 0; s < NKS; ++s) {
     const int d = 16 * s + 8 * hh;
@@ -398,9 +443,12 @@ attn_bwd_dkdv(const BwdParams p) {
       x = *(const u32x4*)(kg + (int64_t)key * p.k_s + d);
       y = *(const u32x4*)(vg + (int64_t)key * p.v_s + d);
     }
-    kf[s] = x ^ p.sign;
+    if (s < NKS - KP)
+      kf[s < NKS - KP ? s : 0] = x ^ p.sign;
+    else
+      kp[(s - (NKS - KP)) * 256] = x ^ p.sign;
     if constexpr (VLDS)
-      *(u32x4*)(vrow + 16 * s) = y;
+      vp[s * 256] = y;
     else
       vf[s] = y;
   }
@@ -472,8 +520,8 @@ attn_bwd_dkdv(const BwdParams p) {
   };
   auto put = [&](int slot) {
     uint16_t* base = lds + slot * 2 * BQ * RS;
-    lq.store(base, xq);
-    ldo.store(base + BQ * RS, xd);
+    lq.template store<RS>(base, xq);
+    ldo.template store<RS>(base + BQ * RS, xd);
     if (tid < BQ) {
       // rows that saw no key in the forward (lse = -inf): P = 0
       lsd[slot][0][tid] = xl > -INFINITY ? -(xl * kLog2e) * inv_c : -INFINITY;
@@ -557,12 +605,14 @@ attn_bwd_dkdv(const BwdParams p) {
           }
         }
 #pragma unroll
-      for (int st = 0; st < NKS; ++st) s = Elt<T>::mma(*(const u32x4*)(qs + a_rd[st]), kf[st], s);
+      for (int st = 0; st < NKS; ++st)
+        s = Elt<T>::mma(*(const u32x4*)(qs + a_rd[st]), st < NKS - KP ? kf[st < NKS - KP ? st : 0] : kp[(st - (NKS - KP)) * 256],
+                        s);
 #pragma unroll
       for (int st = 0; st < NKS; ++st) {
         u32x4 vb;
         if constexpr (VLDS)
-          vb = *(const u32x4*)(vrow + 16 * st);
+          vb = vp[st * 256];
         else
           vb = vf[st];
         dp = Elt<T>::mma(*(const u32x4*)(dos + a_rd[st]), vb, dp);
@@ -610,7 +660,7 @@ attn_bwd_dkdv(const BwdParams p) {
 }
 
 // ---- Sums of split sweeps' partials, in part order (the same result on every
-// run): vector i4 (4 columns) of one or two outputs (b.out null: one).
+// run): vector i4 (4 columns) of one output.
 template <typename T>
 __device__ __forceinline__ void part_sum_store(const PartSum& a, int64_t i4) {
   const int64_t row = i4 * 4 / a.D;
@@ -634,12 +684,20 @@ __device__ __forceinline__ void part_sum_store(const PartSum& a, int64_t i4) {
   }
 }
 
+// dK and dV (same rows) in workgroups [0, kv_wgs), dQ in the rest; an output
+// without partials has no rows.
 template <typename T>
-__global__ void __launch_bounds__(256) attn_bwd_part_sum(const PartSum a, const PartSum b) {
-  const int64_t i4 = (int64_t)block_x() * 256 + thread_x();
-  if (i4 >= a.rows * a.D / 4) return;
-  part_sum_store<T>(a, i4);
-  if (b.out) part_sum_store<T>(b, i4);
+__global__ void __launch_bounds__(256) attn_bwd_part_sum(const PartSum k, const PartSum v, const PartSum q, int kv_wgs) {
+  const int wg = block_x();
+  if (wg < kv_wgs) {
+    const int64_t i4 = (int64_t)wg * 256 + thread_x();
+    if (i4 >= k.rows * k.D / 4) return;
+    part_sum_store<T>(k, i4);
+    part_sum_store<T>(v, i4);
+  } else {
+    const int64_t i4 = (int64_t)(wg - kv_wgs) * 256 + thread_x();
+    if (i4 < q.rows * q.D / 4) part_sum_store<T>(q, i4);
+  }
 }
 
 // ---- Sums of a split tail's block-indexed partials ([ns][blocks][128][D]),
@@ -650,7 +708,8 @@ template <typename T, bool KV>
 __global__ void __launch_bounds__(256) attn_bwd_tail_sum(const BwdParams p) {
   const int D = p.D, ns = KV ? p.nsplit : p.nsplit_q, nfull = KV ? p.nfull : p.nfull_q;
   const int heads = KV ? p.Hkv : p.H;
-  const int64_t nsb = (int64_t)p.B * heads * p.n_blk - nfull;
+  const int n_blk = KV ? p.n_blk : p.n_blk_q;
+  const int64_t nsb = (int64_t)p.B * heads * n_blk - nfull;
   const int64_t i4 = (int64_t)block_x() * 256 + thread_x();
   if (i4 >= nsb * 128 * D / 4) return;
   const int64_t row = i4 * 4 / D;
@@ -658,10 +717,10 @@ __global__ void __launch_bounds__(256) attn_bwd_tail_sum(const BwdParams p) {
   const int sbi = (int)(row / 128), rl = (int)(row - (int64_t)sbi * 128);
   int bh, blk;
   if (KV) {
-    kv_tile(nfull + sbi, p.B * heads, p.n_blk, false, bh, blk);
+    kv_tile(nfull + sbi, p.B * heads, n_blk, false, bh, blk);
   } else {
     FwdParams fp;
-    fp.B = p.B; fp.H = p.H; fp.n_qblk = p.n_blk; fp.n_wg = p.B * p.H * p.n_blk;
+    fp.B = p.B; fp.H = p.H; fp.n_qblk = n_blk; fp.n_wg = p.B * p.H * n_blk;
     wg_tile(nfull + sbi, fp, false, bh, blk);
   }
   const int s = blk * 128 + rl;
@@ -688,44 +747,54 @@ __global__ void __launch_bounds__(256) attn_bwd_tail_sum(const BwdParams p) {
   }
 }
 
-// Launch the sums of the dK/dV partials (sweeps split nsplit ways) or of the
-// dQ partials (nsplit_q ways) that a launch's split sweeps left (errors show
-// in the caller's final hipGetLastError).
+// Launch the sums of the dK/dV partials (kv) and of the dQ partials (q) that a
+// launch's split sweeps left (errors show in the caller's final
+// hipGetLastError).
 template <typename T>
-void launch_part_sums(const BwdParams& p, bool dkdv, hipStream_t s) {
-  PartSum a = {}, b = {};
-  if (dkdv) {
+void launch_part_sums(const BwdParams& p, bool kv, bool q, hipStream_t s) {
+  PartSum dk = {}, dv = {}, dq = {};
+  if (kv) {
     const int64_t rows = (int64_t)p.B * p.Hkv * p.Sk;
-    a = PartSum{p.part, p.dk, p.dk_b, p.dk_h, p.dk_s, rows, p.Hkv, p.Sk, p.D, p.nsplit, p.scale};
-    b = PartSum{p.part + (int64_t)p.nsplit * rows * p.D, p.dv, p.dv_b, p.dv_h, p.dv_s, rows, p.Hkv, p.Sk, p.D,
-                p.nsplit, 1.f};
-  } else {
-    const int64_t rows = (int64_t)p.B * p.H * p.Sq;
-    a = PartSum{p.part_q, p.dq, p.dq_b, p.dq_h, p.dq_s, rows, p.H, p.Sq, p.D, p.nsplit_q, p.scale};
+    dk = PartSum{p.part, p.dk, p.dk_b, p.dk_h, p.dk_s, rows, p.Hkv, p.Sk, p.D, p.nsplit, p.scale};
+    dv = PartSum{p.part + (int64_t)p.nsplit * rows * p.D, p.dv, p.dv_b, p.dv_h, p.dv_s, rows, p.Hkv, p.Sk, p.D,
+                 p.nsplit, 1.f};
   }
-  const int64_t n4 = a.rows * a.D / 4;
-  hipLaunchKernelGGL(attn_bwd_part_sum<T>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a, b);
+  if (q) {
+    const int64_t rows = (int64_t)p.B * p.H * p.Sq;
+    dq = PartSum{p.part_q, p.dq, p.dq_b, p.dq_h, p.dq_s, rows, p.H, p.Sq, p.D, p.nsplit_q, p.scale};
+  }
+  auto wgs = [](const PartSum& a) { return (a.rows * a.D / 4 + 255) / 256; };
+  const int64_t nkv = wgs(dk), n = nkv + wgs(dq);
+  if (n > 0) hipLaunchKernelGGL(attn_bwd_part_sum<T>, dim3((unsigned)n), dim3(256), 0, s, dk, dv, dq, (int)nkv);
 }
 
 // ---- dQ for one block of 128 queries (4 waves x 32 queries), sweeping the
 // key tiles (32 rows of K and V) through double-buffered LDS.
-template <typename T, int DK, bool CAUSAL, bool MASK>
-__global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(DK <= 64 ? (MASK ? 2 : 3) : (DK > 128 || (MASK && CAUSAL)) ? 1 : 2)))
-attn_bwd_dq(const BwdParams p) {
-  constexpr int BQ = 128, BK = 32;
-  constexpr int RS = bwd_lds_stride(DK);
-  constexpr int NKS = DK / 16, NDB = DK / 32;
-  static_assert(DK % 32 == 0, "head-dim bucket");
-  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 2 * BK * RS];  // [slot][K, V][row][col]
+template <int DK, bool CAUSAL, bool MASK>
+struct BwdDq {
+  static constexpr int BQ = 128, BK = 32;
+  static constexpr int RS = bwd_lds_stride(DK);
+  static constexpr int OCC = DK <= 64 ? (MASK && CAUSAL ? 2 : 3) : (DK > 128 || (MASK && CAUSAL)) ? 1 : 2;
   // D > 64 masked non-causal: the dO operands live in LDS (each lane reads
   // back only what it wrote; no barrier), which leaves room for 2 waves per
   // SIMD instead of 1 (masked backward 473 -> 419 us on bf16
   // [2,16,2048,128]; the causal variant would spill 16 registers and gains
   // nothing, so it keeps its registers and 1 wave)
-  constexpr bool DLDS = DK > 64 && DK <= 128 && MASK && !CAUSAL;
-  constexpr int RSD = DK + 8;
-  __shared__ __attribute__((aligned(16))) uint16_t dpark[DLDS ? BQ * RSD : 8];
+  static constexpr bool DLDS = DK > 64 && DK <= 128 && MASK && !CAUSAL;
+  static constexpr int RSD = DK + 8;
+  static constexpr int TILES = 2 * 2 * BK * RS;       // halves: [slot][K, V][row][col]
+  static constexpr int PARK = DLDS ? BQ * RSD : 8;    // halves
+};
+
+// Workgroup `wg` of the dQ sweeps; its LDS arrays (BwdDq's sizes).
+template <typename T, int DK, bool CAUSAL, bool MASK>
+__device__ __forceinline__ void bwd_dq_block(const BwdParams& p, const int wg, uint16_t* const lds,
+                                             uint16_t* const dpark) {
+  using Cfg = BwdDq<DK, CAUSAL, MASK>;
+  constexpr int BQ = Cfg::BQ, BK = Cfg::BK, RS = Cfg::RS, RSD = Cfg::RSD;
+  constexpr bool DLDS = Cfg::DLDS;
+  constexpr int NKS = DK / 16, NDB = DK / 32;
+  static_assert(DK % 32 == 0, "head-dim bucket");
 
   const int tid = thread_x(), wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   // split sweeps: (query block, part) pairs as ns virtual blocks per block
@@ -734,7 +803,7 @@ attn_bwd_dq(const BwdParams p) {
   if (!CAUSAL && p.nfull_q > 0) {
     // split tail: the first nfull_q workgroups take whole blocks, the rest
     // ns-way parts of the remaining blocks
-    const int w = block_x();
+    const int w = wg;
     int lb = w;
     part = 0;
     if (w >= p.nfull_q) {
@@ -746,13 +815,13 @@ attn_bwd_dq(const BwdParams p) {
       ns = 1;
     }
     FwdParams fp;
-    fp.B = p.B; fp.H = p.H; fp.n_qblk = p.n_blk; fp.n_wg = p.B * p.H * p.n_blk;
+    fp.B = p.B; fp.H = p.H; fp.n_qblk = p.n_blk_q; fp.n_wg = p.B * p.H * p.n_blk_q;
     wg_tile(lb, fp, false, bh, qblk);
   } else {
     FwdParams fp;
-    fp.B = p.B; fp.H = p.H; fp.n_qblk = p.n_blk * ns; fp.n_wg = p.n_wg;
+    fp.B = p.B; fp.H = p.H; fp.n_qblk = p.n_blk_q * ns; fp.n_wg = p.n_wg_q;
     int vblk;
-    wg_tile(block_x(), fp, CAUSAL, bh, vblk);  // causal: longest key sweeps first
+    wg_tile(wg, fp, CAUSAL, bh, vblk);  // causal: longest key sweeps first
     qblk = vblk / ns;
     part = vblk - qblk * ns;
   }
@@ -828,8 +897,8 @@ attn_bwd_dq(const BwdParams p) {
   };
   auto put = [&](int slot) {
     uint16_t* base = lds + slot * 2 * BK * RS;
-    lk.store(base, xk);
-    lv.store(base + BK * RS, xv);
+    lk.template store<RS>(base, xk);
+    lv.template store<RS>(base + BK * RS, xv);
   };
 
   const float c = p.c;
@@ -929,7 +998,7 @@ attn_bwd_dq(const BwdParams p) {
   }
 
   if (ns > 1 && sb >= 0) {  // split tail: block-indexed partial rows, unscaled
-    const int64_t nsb = (int64_t)p.B * p.H * p.n_blk - p.nfull_q;
+    const int64_t nsb = (int64_t)p.B * p.H * p.n_blk_q - p.nfull_q;
     store_rows_f32<NDB>(p.part_q + ((int64_t)part * nsb + sb) * BQ * D, qrow - qblk * BQ, Sq - qblk * BQ, D, hh,
                         dqa);
     return;
@@ -940,6 +1009,38 @@ attn_bwd_dq(const BwdParams p) {
   }
   uint16_t* dqg = (uint16_t*)p.dq + b * p.dq_b + h * p.dq_h;
   store_rows<T, NDB>(dqg, p.dq_s, qrow, Sq, D, hh, dqa, p.scale);
+}
+
+// ---- The gradient sweeps, both in one launch: the dK/dV workgroups (p.n_wg of
+// them, the longer ones) first, then the dQ workgroups.  Neither sweep needs
+// the other's result, so a grid of few workgroups fills the CUs that one sweep
+// alone leaves idle, and a large one runs into the other's blocks instead of a
+// tail.  Against a launch each, same MI355X run, whole backward: bf16 causal
+// [2,16,512,512,128] 58.5 -> 39.6 us, [2,10,4096,4096,128] 419 -> 355,
+// [2,10,2048,2048,256] 652 -> 454 not causal.
+enum : int { BWD_BOTH, BWD_DKDV, BWD_DQ };
+
+template <int DK, bool CAUSAL, bool MASK, int SWEEP>
+constexpr int bwd_occ() {
+  const int kv = BwdDkdv<DK, CAUSAL, MASK>::OCC, q = BwdDq<DK, CAUSAL, MASK>::OCC;
+  return SWEEP == BWD_DKDV ? kv : SWEEP == BWD_DQ ? q : kv < q ? kv : q;
+}
+
+template <typename T, int DK, bool CAUSAL, bool MASK, int SWEEP>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_occ<DK, CAUSAL, MASK, SWEEP>())))
+attn_bwd_grads(const BwdParams p) {
+  using A = BwdDkdv<DK, CAUSAL, MASK>;
+  using Q = BwdDq<DK, CAUSAL, MASK>;
+  static_assert(A::TILES == Q::TILES, "the sweeps share the tile slots");
+  constexpr int PARK = SWEEP == BWD_DQ ? Q::PARK : SWEEP == BWD_DKDV || A::PARK > Q::PARK ? A::PARK : Q::PARK;
+  __shared__ __attribute__((aligned(16))) uint16_t lds[A::TILES];
+  __shared__ __attribute__((aligned(16))) uint16_t park[PARK];
+  __shared__ __attribute__((aligned(16))) float lsd[SWEEP == BWD_DQ ? 4 : A::LSD];
+  const int wg = block_x();
+  if (SWEEP == BWD_DKDV || (SWEEP == BWD_BOTH && wg < p.n_wg))
+    bwd_dkdv_block<T, DK, CAUSAL, MASK>(p, wg, lds, park, lsd);
+  else
+    bwd_dq_block<T, DK, CAUSAL, MASK>(p, SWEEP == BWD_BOTH ? wg - p.n_wg : wg, lds, park);
 }
 
 }  // namespace cmpext3

@@ -1,8 +1,8 @@
 // Launch sequence of the attention backward (templates in attn_bwd16.h):
-// Delta, then dK/dV over key blocks (split sweeps: then the sum of their
-// partials), then dQ over query blocks, all on the caller's stream.  Head
-// dims up to 64 use the 64 bucket, up to 128 the 128 bucket, up to 192 and
-// 256 those (columns past D are zero in every operand and never stored).
+// Delta, then dK/dV over key blocks and dQ over query blocks in one launch, then
+// the sums of what split sweeps left, all on the caller's stream.  Head dims up
+// to 64 use the 64 bucket, up to 128 the 128 bucket, up to 192 and 256 those
+// (columns past D are zero in every operand and never stored).
 #include "attn_bwd16.h"
 
 namespace cmpext3 {
@@ -20,30 +20,31 @@ hipError_t launch_bwd_t(const BwdParams& p0, hipStream_t s) {
   if (ns == 1 || CAUSAL) p.nfull = 0;
   const int n_kv = p.B * p.Hkv * p.n_blk;
   p.n_wg = p.nfull > 0 ? p.nfull + (n_kv - p.nfull) * ns : n_kv * ns;
-  hipLaunchKernelGGL((attn_bwd_dkdv<T, DK, CAUSAL, MASK>), dim3(p.n_wg), dim3(256), 0, s, p);
-  if (ns > 1) {
-    if (p.nfull > 0) {
-      const int64_t n4 = (int64_t)(n_kv - p.nfull) * 128 * p.D / 4;
-      hipLaunchKernelGGL((attn_bwd_tail_sum<T, true>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, p);
-    } else {
-      launch_part_sums<T>(p, true, s);
-    }
-  }
-  p.n_blk = (p.Sq + 127) / 128;
+  p.n_blk_q = (p.Sq + 127) / 128;
   const int nsq = p.nsplit_q > 1 && p.part_q ? p.nsplit_q : 1;
   p.nsplit_q = nsq;
   if (nsq == 1 || CAUSAL) p.nfull_q = 0;
-  const int n_q = p.B * p.H * p.n_blk;
-  p.n_wg = p.nfull_q > 0 ? p.nfull_q + (n_q - p.nfull_q) * nsq : n_q * nsq;
-  hipLaunchKernelGGL((attn_bwd_dq<T, DK, CAUSAL, MASK>), dim3(p.n_wg), dim3(256), 0, s, p);
-  if (nsq > 1) {
-    if (p.nfull_q > 0) {
-      const int64_t n4 = (int64_t)(n_q - p.nfull_q) * 128 * p.D / 4;
-      hipLaunchKernelGGL((attn_bwd_tail_sum<T, false>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, p);
-    } else {
-      launch_part_sums<T>(p, false, s);
+  const int n_q = p.B * p.H * p.n_blk_q;
+  p.n_wg_q = p.nfull_q > 0 ? p.nfull_q + (n_q - p.nfull_q) * nsq : n_q * nsq;
+  bool apart = false;
+  if constexpr (DK == 64 && CAUSAL) {
+    apart = last_round_full(n_kv, (int64_t)BwdDkdv<DK, CAUSAL, MASK>::OCC * device_cus());
+    if (apart) {
+      hipLaunchKernelGGL((attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_DKDV>), dim3(p.n_wg), dim3(256), 0, s, p);
+      hipLaunchKernelGGL((attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_DQ>), dim3(p.n_wg_q), dim3(256), 0, s, p);
     }
   }
+  if (!apart)
+    hipLaunchKernelGGL((attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_BOTH>), dim3(p.n_wg + p.n_wg_q), dim3(256), 0, s, p);
+  if (p.nfull > 0) {
+    const int64_t n4 = (int64_t)(n_kv - p.nfull) * 128 * p.D / 4;
+    hipLaunchKernelGGL((attn_bwd_tail_sum<T, true>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, p);
+  }
+  if (p.nfull_q > 0) {
+    const int64_t n4 = (int64_t)(n_q - p.nfull_q) * 128 * p.D / 4;
+    hipLaunchKernelGGL((attn_bwd_tail_sum<T, false>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, p);
+  }
+  launch_part_sums<T>(p, ns > 1 && p.nfull == 0, nsq > 1 && p.nfull_q == 0, s);
   return hipGetLastError();
 }
 
@@ -79,10 +80,11 @@ BwdSplit bwd16_split(int B, int H, int Hkv, int Sq, int Sk, int D, bool causal, 
   const int64_t n_kv = (int64_t)B * Hkv * ((Sk + 127) / 128), n_q = (int64_t)B * H * ((Sq + 127) / 128);
   const int64_t t_kv = (int64_t)(H / Hkv) * ((Sq + 31) / 32), t_q = (Sk + 31) / 32;
   // us per 32-row tile of one block, a CU to itself
+  const float mx = masked ? 1.7f : 1.f;
   const float us_kv = dk <= 64 ? 0.74f : dk <= 128 ? 1.2f : dk <= 192 ? 2.f : 2.8f;
   const float us_q = dk <= 64 ? 0.49f : dk <= 128 ? 0.86f : dk <= 192 ? 1.35f : 1.83f;
-  sp.ns_kv = split_sweep(n_kv, occ_kv, cus, causal, t_kv, us_kv, 8e-6f * B * Hkv * Sk * D);
-  sp.ns_q = split_sweep(n_q, occ_q, cus, causal, t_q, us_q, 4e-6f * B * H * Sq * D);
+  sp.ns_kv = split_sweep(n_kv, occ_kv, cus, causal, t_kv, mx * us_kv, 8e-6f * B * Hkv * Sk * D);
+  sp.ns_q = split_sweep(n_q, occ_q, cus, causal, t_q, mx * us_q, 4e-6f * B * H * Sq * D);
   // non-causal grids past one round: split only the last, partial round
   if (!causal && sp.ns_kv == 1) sp.ns_kv = split_tail(n_kv, occ_kv, cus, t_kv, &sp.nfull_kv);
   if (!causal && sp.ns_q == 1) sp.ns_q = split_tail(n_q, occ_q, cus, t_q, &sp.nfull_q);

@@ -6,8 +6,8 @@
 // The same gradients as the fp16/bf16 backward (attn_bwd16.h), with
 // P = exp2(S * c - lse * log2 e) rebuilt from the forward's row log-sum-exp:
 //   Delta_i = sum_d dO_id O_id                     (attn_bwd32_delta)
-//   dV = P^T dO,  dK = scale * dS^T Q              (attn_bwd32_dkdv, per 64 keys)
-//   dQ = scale * dS K                              (attn_bwd32_dq, per 64 queries)
+//   dV = P^T dO,  dK = scale * dS^T Q              (per 64 keys)
+//   dQ = scale * dS K                              (per 64 queries)
 //   with dP = dO V^T and dS = P * (dP - Delta).
 // Each gradient row is written by exactly one workgroup (no atomics), so the
 // results are bit-identical from run to run.
@@ -157,17 +157,17 @@ __device__ __forceinline__ void store_rows32(float* base, int64_t row_stride, in
 // per tile.  Grouped-query K/V: the sweep runs over every query head of the
 // K/V head's group, so the group's contributions add up in registers.
 template <int DK, bool CAUSAL>
-__global__ void __launch_bounds__(256) attn_bwd32_dkdv(const BwdParams p) {
+__device__ __forceinline__ void bwd32_dkdv_block(const BwdParams& p, const int wg, float* const lds,
+                                                 float* const lsdp) {
   constexpr int BQ = 32, BKV = 64;
   constexpr int NKS = DK / 4;            // k-steps of S and dP
   constexpr int NDB = (DK + 15) / 16;    // 16-column blocks of dK and dV
   constexpr int CW = NDB * 16;           // tile columns (zero past D)
   using Tile = Tile32<BQ, CW>;
   constexpr int RS = Tile::RS;
-  __shared__ __attribute__((aligned(16))) float lds[2 * 2 * BQ * RS];  // [slot][Q, dO][row][col]
   // [slot][lse2, Delta][row]: lse2 = lse * log2 e (+inf for rows past Sq or
   // rows that saw no key: P = 0 there)
-  __shared__ __attribute__((aligned(16))) float lsd[2][2][BQ];
+  float (*const lsd)[2][BQ] = (float (*)[2][BQ])lsdp;
 
   const int tid = thread_x(), wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   // (batch, K/V head) and key block; split sweeps: (block, part) pairs as
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) attn_bwd32_dkdv(const BwdParams p) {
   int bhk, kb, part;
   {
     int bh0, vb;
-    kv_tile(block_x(), p.B * p.Hkv, p.n_blk * ns, CAUSAL, bh0, vb);
+    kv_tile(wg, p.B * p.Hkv, p.n_blk * ns, CAUSAL, bh0, vb);
     bhk = __builtin_amdgcn_readfirstlane(bh0);
     vb = __builtin_amdgcn_readfirstlane(vb);
     kb = __builtin_amdgcn_readfirstlane(vb / ns);
@@ -363,14 +363,13 @@ __global__ void __launch_bounds__(256) attn_bwd32_dkdv(const BwdParams p) {
 // ---- dQ for one block of 64 queries (4 waves x 16 queries), sweeping
 // 32-key tiles of K and V through double-buffered LDS.
 template <int DK, bool CAUSAL>
-__global__ void __launch_bounds__(256) attn_bwd32_dq(const BwdParams p) {
+__device__ __forceinline__ void bwd32_dq_block(const BwdParams& p, const int wg, float* const lds) {
   constexpr int BQ = 64, BK = 32;
   constexpr int NKS = DK / 4;
   constexpr int NDB = (DK + 15) / 16;
   constexpr int CW = NDB * 16;
   using Tile = Tile32<BK, CW>;
   constexpr int RS = Tile::RS;
-  __shared__ __attribute__((aligned(16))) float lds[2 * 2 * BK * RS];  // [slot][K, V][row][col]
 
   const int tid = thread_x(), wave = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   // split sweeps: (query block, part) pairs as ns virtual blocks per block
@@ -378,9 +377,9 @@ __global__ void __launch_bounds__(256) attn_bwd32_dq(const BwdParams p) {
   int bh, qblk, part;
   {
     FwdParams fp;
-    fp.B = p.B; fp.H = p.H; fp.n_qblk = p.n_blk * ns; fp.n_wg = p.n_wg;
+    fp.B = p.B; fp.H = p.H; fp.n_qblk = p.n_blk_q * ns; fp.n_wg = p.n_wg_q;
     int vblk;
-    wg_tile(block_x(), fp, CAUSAL, bh, vblk);  // causal: longest key sweeps first
+    wg_tile(wg, fp, CAUSAL, bh, vblk);  // causal: longest key sweeps first
     qblk = vblk / ns;
     part = vblk - qblk * ns;
   }
@@ -506,6 +505,20 @@ __global__ void __launch_bounds__(256) attn_bwd32_dq(const BwdParams p) {
   store_rows32<NDB>(dqg, p.dq_s, qrow, Sq, D, g, dqa, p.scale);
 }
 
+// ---- Both sweeps in one launch, dK/dV first, as in attn_bwd16.h
+template <int DK, bool CAUSAL, int SWEEP>
+__global__ void __launch_bounds__(256) attn_bwd32_grads(const BwdParams p) {
+  constexpr int ROWS = 32;                                               // of a Q/dO or K/V tile
+  constexpr int TILES = 2 * 2 * ROWS * Tile32<ROWS, (DK + 15) / 16 * 16>::RS;  // floats: [slot][2][row][col]
+  __shared__ __attribute__((aligned(16))) float lds[TILES];
+  __shared__ __attribute__((aligned(16))) float lsd[SWEEP == BWD_DQ ? 4 : 2 * 2 * ROWS];
+  const int wg = block_x();
+  if (SWEEP == BWD_DKDV || (SWEEP == BWD_BOTH && wg < p.n_wg))
+    bwd32_dkdv_block<DK, CAUSAL>(p, wg, lds, lsd);
+  else
+    bwd32_dq_block<DK, CAUSAL>(p, SWEEP == BWD_BOTH ? wg - p.n_wg : wg, lds);
+}
+
 template <int DK, bool CAUSAL>
 hipError_t launch_bwd32_t(const BwdParams& p0, hipStream_t s) {
   BwdParams p = p0;
@@ -514,15 +527,25 @@ hipError_t launch_bwd32_t(const BwdParams& p0, hipStream_t s) {
   p.n_blk = (p.Sk + 63) / 64;
   const int ns = p.nsplit > 1 && p.part ? p.nsplit : 1;
   p.nsplit = ns;
-  p.n_wg = p.B * p.Hkv * p.n_blk * ns;
-  hipLaunchKernelGGL((attn_bwd32_dkdv<DK, CAUSAL>), dim3(p.n_wg), dim3(256), 0, s, p);
-  if (ns > 1) launch_part_sums<float>(p, true, s);
-  p.n_blk = (p.Sq + 63) / 64;
+  const int n_kv = p.B * p.Hkv * p.n_blk;
+  p.n_wg = n_kv * ns;
+  p.n_blk_q = (p.Sq + 63) / 64;
   const int nsq = p.nsplit_q > 1 && p.part_q ? p.nsplit_q : 1;
   p.nsplit_q = nsq;
-  p.n_wg = p.B * p.H * p.n_blk * nsq;
-  hipLaunchKernelGGL((attn_bwd32_dq<DK, CAUSAL>), dim3(p.n_wg), dim3(256), 0, s, p);
-  if (nsq > 1) launch_part_sums<float>(p, false, s);
+  p.n_wg_q = p.B * p.H * p.n_blk_q * nsq;
+  // these two dQ sweeps run a wave per SIMD more by themselves
+  bool apart = false;
+  if constexpr (DK == (CAUSAL ? 32 : 40)) {
+    const int cus = device_cus();
+    apart = n_kv >= 2 * cus && last_round_full(n_kv, cus);
+    if (apart) {
+      hipLaunchKernelGGL((attn_bwd32_grads<DK, CAUSAL, BWD_DKDV>), dim3(p.n_wg), dim3(256), 0, s, p);
+      hipLaunchKernelGGL((attn_bwd32_grads<DK, CAUSAL, BWD_DQ>), dim3(p.n_wg_q), dim3(256), 0, s, p);
+    }
+  }
+  if (!apart)
+    hipLaunchKernelGGL((attn_bwd32_grads<DK, CAUSAL, BWD_BOTH>), dim3(p.n_wg + p.n_wg_q), dim3(256), 0, s, p);
+  launch_part_sums<float>(p, ns > 1, nsq > 1, s);
   return hipGetLastError();
 }
 
