@@ -540,7 +540,9 @@ attn_fwd_mfma16(const FwdParams p, const SplitArgs sa) {
           }
       };
       // Raise the offset to the tile's row max (never lower it after the first
-      // live tile); rescale O and l by 2^-delta.  Returns delta.
+      // live tile); rescale O and l by 2^-delta, at most 1 (only that tile's
+      // delta can be negative, O and l are zero up to it, and 2^-delta is
+      // infinite from -128 down).  Returns delta.
       auto rescale_to_max = [&]() {
         float mq = -INFINITY;
 #pragma unroll
@@ -550,7 +552,7 @@ attn_fwd_mfma16(const FwdParams p, const SplitArgs sa) {
         const float mx = xhalf_max(mq);
         float delta = first[qb] ? mx : fmaxf(mx, 0.f);
         if (mx == -INFINITY) delta = 0.f;
-        const float alpha = fast_exp2(-delta);
+        const float alpha = fast_exp2(-fmaxf(delta, 0.f));
         mb[qb] += delta;
         lsum[qb] *= alpha;
 #pragma unroll

@@ -717,12 +717,14 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
   static_assert(NCH % 2 == 0, "chunk split");
 
   // Raise the offset to the row max mx (never lower it once a live key was
-  // seen) and rescale O and l; returns the shift applied to the scores.
+  // seen) and rescale O and l; returns the shift applied to the scores.  Only
+  // the first live tile's delta can be negative, and O and l are zero up to it:
+  // they are scaled by at most 1 (2^-delta is infinite from -128 down).
   auto rescale = [&](float mx) {
     const bool fst = thr == -INFINITY;
     float delta = fst ? mx : fmaxf(mx, 0.f);
     if (mx == -INFINITY) delta = 0.f;
-    const float alpha = fast_exp2(-delta);
+    const float alpha = fast_exp2(-fmaxf(delta, 0.f));
     mb += delta;
     ls *= alpha;
 #pragma unroll
