@@ -265,7 +265,11 @@ struct TileLoader {
   // load's scalar offset), or, where a pass is no whole number of rows (DK =
   // 192), 64-column strips: either way one address register, one LDS offset.
   // With one of each per chunk the dK/dV sweep at DK = 128 spilled some of them
-  // and waited for the whole fetch to reload them.
+  // and waited for the whole fetch to reload them.  The scalar offset stays
+  // within the buffer's `range` bytes: the bounds check compares the vector
+  // offset with range minus the scalar one, so a pass that starts past the last
+  // row (S = 333 at DK = 128: its second pass starts at row 336) is given
+  // exactly `range`, where nothing is in bounds and every row reads zero.
   static constexpr bool BYROW = 256 % KCH == 0;
   static constexpr int RPP = BYROW ? 256 / KCH : 0;  // rows a pass
   int voff, loff, step, room;
@@ -277,11 +281,13 @@ struct TileLoader {
     step = (int)(RPP * row_stride * 2);
     room = D - 8 * c8;  // columns left from this thread's first chunk on
   }
-  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int soff, u32x4 (&x)[N]) const {
+  // soff: byte offset of the tile's first row, below range
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t range, int soff, u32x4 (&x)[N]) const {
 #pragma unroll
     for (int it = 0; it < N; ++it)
       x[it] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, BYROW ? voff : voff + 128 * it, soff + it * step, 0));
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, BYROW ? voff : voff + 128 * it,
+                                                       BYROW && it > 0 ? (int)min((uint32_t)(soff + it * step), range) : soff, 0));
   }
   template <int RS>
   __device__ __forceinline__ void store(uint16_t* dst, const u32x4 (&x)[N]) const {
@@ -495,11 +501,12 @@ __device__ __forceinline__ void bwd_dkdv_block(const BwdParams& p, const int wg,
     const int h = h0 + fg;
     const uint16_t* qg = (const uint16_t*)p.q + b * p.q_b + h * p.q_h;
     const uint16_t* dog = (const uint16_t*)p.dout + b * p.do_b + h * p.do_h;
-    const __amdgpu_buffer_rsrc_t qrs = uniform_rsrc(qg, ((int64_t)(Sq - 1) * p.q_s + D) * 2);
-    const __amdgpu_buffer_rsrc_t dors = uniform_rsrc(dog, ((int64_t)(Sq - 1) * p.do_s + D) * 2);
+    const int64_t qn = ((int64_t)(Sq - 1) * p.q_s + D) * 2, don = ((int64_t)(Sq - 1) * p.do_s + D) * 2;
+    const __amdgpu_buffer_rsrc_t qrs = uniform_rsrc(qg, qn);
+    const __amdgpu_buffer_rsrc_t dors = uniform_rsrc(dog, don);
     const int q0 = ft * BQ;
-    lq.load(qrs, (int)(q0 * p.q_s * 2), xq);
-    ldo.load(dors, (int)(q0 * p.do_s * 2), xd);
+    lq.load(qrs, (uint32_t)qn, (int)(q0 * p.q_s * 2), xq);
+    ldo.load(dors, (uint32_t)don, (int)(q0 * p.do_s * 2), xd);
     // this head's lse / Delta rows; used only in put(), so the loads are not
     // waited for before the current tile's products
     const int64_t hoff = ((int64_t)b * p.H + h) * Sq;
@@ -863,8 +870,9 @@ __device__ __forceinline__ void bwd_dq_block(const BwdParams& p, const int wg, u
   const int hk = h / p.group;
   const uint16_t* kg = (const uint16_t*)p.k + b * p.k_b + hk * p.k_h;
   const uint16_t* vg = (const uint16_t*)p.v + b * p.v_b + hk * p.v_h;
-  const __amdgpu_buffer_rsrc_t krs = uniform_rsrc(kg, ((int64_t)(Sk - 1) * p.k_s + D) * 2);
-  const __amdgpu_buffer_rsrc_t vrs = uniform_rsrc(vg, ((int64_t)(Sk - 1) * p.v_s + D) * 2);
+  const int64_t kn = ((int64_t)(Sk - 1) * p.k_s + D) * 2, vn = ((int64_t)(Sk - 1) * p.v_s + D) * 2;
+  const __amdgpu_buffer_rsrc_t krs = uniform_rsrc(kg, kn);
+  const __amdgpu_buffer_rsrc_t vrs = uniform_rsrc(vg, vn);
   TileLoader<DK> lk, lv;
   lk.init(tid, p.k_s, D, RS);
   lv.init(tid, p.v_s, D, RS);
@@ -892,8 +900,8 @@ __device__ __forceinline__ void bwd_dq_block(const BwdParams& p, const int wg, u
   const int wlast = qblk * BQ + wave * 32 + 31;            // this wave's last query
   u32x4 xk[TileLoader<DK>::N], xv[TileLoader<DK>::N];
   auto fetch = [&](int t) {
-    lk.load(krs, (int)(t * BK * p.k_s * 2), xk);
-    lv.load(vrs, (int)(t * BK * p.v_s * 2), xv);
+    lk.load(krs, (uint32_t)kn, (int)(t * BK * p.k_s * 2), xk);
+    lv.load(vrs, (uint32_t)vn, (int)(t * BK * p.v_s * 2), xv);
   };
   auto put = [&](int slot) {
     uint16_t* base = lds + slot * 2 * BK * RS;
