@@ -172,7 +172,9 @@ int cmpext3_attn_fwd_masked(const void* q, const void* k, const void* v, void* o
  * workspace is first used, and every launch leaves them zero when it
  * completes, so one workspace can serve any sequence of calls, of any
  * shapes, that run one after another (for example every call on one
- * stream).  The rest needs no initialisation.  Two launches that may run at
+ * stream, from any thread: the launches of a call are submitted together,
+ * other calls given the same workspace pointer wait for them).  The rest
+ * needs no initialisation.  Two launches that may run at
  * the same time must not share a workspace: they would not hang, but they
  * could mix each other's partial results (wrong output, counters left
  * non-zero for later calls).  The workspace is only read and written by the
@@ -232,7 +234,7 @@ int cmpext3_attn_fwd_plan(int dtype, int B, int H, int H_kv, int Sq, int Sk, int
  * that size (same plan, same result bit for bit).  A split that would need more is cut to
  * fewer key ranges (down to none), so no problem is refused for lack of
  * room.  Every call on one device shares that device's array: calls in
- * stream order are safe; calls that overlap in time on one device (two
+ * stream order are safe, also from several threads; calls that overlap in time on one device (two
  * streams, or a graph replay beside an eager call) must not be made -- they
  * cannot hang (no launch waits for another workgroup), but they can give
  * wrong results and leave counters non-zero, which can make later split

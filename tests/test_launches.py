@@ -1,0 +1,103 @@
+"""What reaches a stream when C entry points are called (no GPU).
+
+The library runs against tests/launch_recorder.cpp, which records launches
+instead of making them, in a process of its own.  Tensors are addresses that
+nothing on the host reads.
+"""
+from __future__ import annotations
+
+import json
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+LIB = HERE.parent / "torch-cmp-patch_amd" / "cmpext3" / "libcmpext3_attn.so"
+
+PRELUDE = """
+import ctypes, json, sys, threading
+rec = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+vp, ci, sz, i64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t, ctypes.c_int64
+lib.cmpext3_attn_bwd_workspace_size.restype = sz
+lib.cmpext3_attn_fwd_workspace_size.restype = sz
+F16, BF16, F32, BOOL = 0, 1, 2, 3
+A = 1 << 32                                     # stands for every tensor
+s3 = lambda *s: (i64 * 3)(*s)
+def fwd(entry, dt, B, H, S, D, mask, ws=None, nbytes=0, causal=0):
+    st = s3(H * S * D, S * D, D)
+    ms = s3(0, 0, S) if mask else s3(0, 0, 0)
+    tail = [vp(A) if mask else None, BOOL if mask else -1, ms, ctypes.c_float(0.1), causal]
+    if entry == "ws":
+        tail += [vp(ws), sz(nbytes), None]
+        f = lib.cmpext3_attn_fwd_ws
+    else:
+        tail += [None]
+        f = lib.cmpext3_attn_fwd_noalloc
+    return f(vp(A), vp(A), vp(A), vp(A), dt, B, H, H, S, S, D, st, st, st, st, *tail)
+def bwd(dt, B, H, Hkv, Sq, Sk, D, causal, ws=None, nbytes=0):
+    q, k = s3(H * Sq * D, Sq * D, D), s3(Hkv * Sk * D, Sk * D, D)
+    return lib.cmpext3_attn_bwd_ws(*[vp(A)] * 10, dt, B, H, Hkv, Sq, Sk, D, q, k, k, q, q, q, k, k, None, -1,
+                                   s3(0, 0, 0), ctypes.c_float(0.1), causal, vp(ws), sz(nbytes), None)
+def launches():
+    out = []
+    for i in range(rec.recorder_count()):
+        name, wg, th = ctypes.c_char_p(), ctypes.c_uint64(), ctypes.c_uint64()
+        tag = rec.recorder_get(i, ctypes.byref(name), ctypes.byref(wg), ctypes.byref(th))
+        out.append((tag, name.value.decode(), wg.value, th.value))
+    return out
+"""
+
+
+@pytest.fixture(scope="module")
+def recorder(tmp_path_factory):
+    so = tmp_path_factory.mktemp("recorder") / "launch_recorder.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-pthread", str(HERE / "launch_recorder.cpp"),
+                    "-o", str(so)], check=True)
+    return so
+
+
+def _run(recorder, body):
+    res = subprocess.run([sys.executable, "-c", PRELUDE + body, str(recorder), str(LIB)], capture_output=True,
+                         text=True, timeout=120)
+    assert res.returncode == 0, res.stderr
+    return json.loads(res.stdout)
+
+
+# Two threads on one stream with one workspace (or the library's fixed one):
+# a bool-masked call makes its mask's bits there and then reads them, so no
+# other call's launch may come between the two.
+@pytest.mark.parametrize("entry,other", [("ws", "masked"), ("ws", "split"), ("ws", "backward"),
+                                         ("noalloc", "masked"), ("noalloc", "split")])
+def test_a_masked_calls_launches_stay_together(recorder, entry, other):
+    got = _run(recorder, f"""
+entry, other = {entry!r}, {other!r}
+rec.recorder_slow(b"attn_mask_bits", 3000)
+n, ws, done, rcs = 1 << 28, 1 << 34, [], set()
+def masked(tag):
+    rec.recorder_tag(tag)
+    for _ in range(8):
+        rcs.add(fwd(entry, BF16, 1, 2, 700, 128, True, ws, n))
+    done.append(tag)
+def second():
+    if other == "masked":
+        return masked(2)
+    rec.recorder_tag(2)
+    while True:
+        rcs.add(fwd(entry, BF16, 1, 8, 1024, 128, False, ws, n) if other == "split"
+                else bwd(BF16, 1, 8, 2, 1024, 1024, 128, 1, ws, n))
+        if done:
+            break
+ts = [threading.Thread(target=masked, args=(1,)), threading.Thread(target=second)]
+[t.start() for t in ts]; [t.join() for t in ts]
+print(json.dumps([sorted(rcs), launches()]))
+""")
+    rcs, seen = got
+    assert rcs == [0]
+    assert {tag for tag, *_ in seen} == {1, 2}
+    bits = [i for i, (_, name, *_) in enumerate(seen) if "attn_mask_bits" in name]
+    assert len(bits) == (16 if other == "masked" else 8)
+    for i in bits:
+        assert seen[i + 1][0] == seen[i][0] and "attn_fwd_pipe16" in seen[i + 1][1], seen[max(0, i - 2):i + 4]

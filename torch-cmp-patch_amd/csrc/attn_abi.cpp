@@ -12,6 +12,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <mutex>
+
 #include "../../include/cmpext3_attn.h"
 #include "attn_common.h"
 
@@ -119,6 +121,18 @@ int piece_bytes(const void* q, const void* k, const void* v, const void* o, int 
   add(v_str, B, H_kv, Sk);
   add(o_str, B, H, Sq);
   return (bits & 15) == 0 ? 16 : (bits & 7) == 0 ? 8 : (bits & 3) == 0 ? 4 : 2;
+}
+
+// Held while a call's launches are submitted.  A call that uses a workspace
+// (or the fixed scratch: null) may take several launches that hand data over
+// through it -- mask bits and the attention that reads them, a backward's
+// partials and their sums -- and another thread's call on the same stream and
+// space must not put a launch in between: stream order alone would then give
+// one call the other's bits.  Calls on different spaces rarely share a lock;
+// calls with no space take none.
+std::mutex& space_lock(const void* space) {
+  static std::mutex locks[64];
+  return locks[((uintptr_t)space * 0x9E3779B97F4A7C15ull) >> 58];
 }
 
 bool strides_nonneg(const int64_t s[3], int n0, int n1, int n2) {
@@ -277,6 +291,8 @@ int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, i
   p.workspace_bytes = workspace ? workspace_bytes : 0;
   p.elem_rows = chunks ? 0 : piece;
 
+  std::unique_lock<std::mutex> submit(space_lock(workspace), std::defer_lock);
+  if (fixed_exchange || p.workspace) submit.lock();
   hipError_t err;
   if (dtype == CMPEXT3_DTYPE_F32)
     err = cmpext3::launch_mfma32(p, causal != 0, stream);
@@ -527,6 +543,8 @@ int cmpext3_attn_bwd_ws(const void* q, const void* k, const void* v, const void*
       p.part_q = (float*)((char*)workspace + used);
     }
   }
+  std::unique_lock<std::mutex> submit(space_lock(workspace), std::defer_lock);
+  if (workspace) submit.lock();
   const hipError_t err = dtype == CMPEXT3_DTYPE_F32
                              ? cmpext3::launch_bwd32(p, causal != 0, stream)
                              : cmpext3::launch_bwd16(p, dtype == CMPEXT3_DTYPE_BF16, causal != 0, stream);
