@@ -15,8 +15,9 @@
  * through a fixed per-device array inside the library.  Every other call, and
  * any call whose workspace is null or too small, runs without the split (or
  * with fewer key ranges): the same result within rounding (a split adds the
- * parts' partial sums in another order, and two-part fp16 splits round each
- * part's O/l to fp16), bit-identical from one call to the next for a given
+ * parts' partial sums in another order, and fp16 splits of grids and sweeps
+ * that allow two parts and no more, and stream-K, round each part's O/l to
+ * fp16), bit-identical from one call to the next for a given
  * plan.  No launch ever waits for another workgroup, so no interleaving of
  * launches can hang the GPU.  All launches go on the stream the caller
  * passes.

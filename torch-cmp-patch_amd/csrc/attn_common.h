@@ -318,6 +318,9 @@ struct SplitArgs {
   // block is a possible split block, nparts the part slots per block);
   // 0 otherwise
   int sk_wgs;
+  // two fp16 parts of the pipelined kernel exchange O / l in fp16 (else, and
+  // three parts and more always, unnormalised O in fp32)
+  int half16;
 };
 
 // float4 vectors each lane of the fp16/bf16 kernels leaves per part: its O

@@ -973,12 +973,12 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     int* const ctr = sa.cnt + 2 * (sb * nwl + wave);  // {parts arrived, states written}
     // a part whose keys are all masked for this row holds nothing: offset -inf
     const float m_own = lsum > 0.f ? mb : -INFINITY;
-    // Two fp16 parts exchange their O normalised by their own row sum, in
-    // fp16 (a quarter of the bytes): 2 * NDB vectors, then (m, l) as 8 bytes
-    // per lane.  Both parts round their own O this way, so the result does
+    // Two fp16 parts, where the plan says so (short blocks: always), exchange
+    // their O normalised by their own row sum, in fp16 (half of the bytes):
+    // 2 * NDB vectors, then (m, l) as 8 bytes per lane.  Both parts round their own O this way, so the result does
     // not depend on which one writes (reruns stay bit-identical); rounding O/l
     // to fp16 before the merge adds at most one fp16 rounding to the output.
-    const bool half_x = std::is_same<T, _Float16>::value && (nparts == 2 || STREAMK);
+    const bool half_x = std::is_same<T, _Float16>::value && (STREAMK || (nparts == 2 && ((OPT & 128) || sa.half16)));
     u32x4 own_h[2 * NDB];  // half_x: this part's O / l in fp16
     if (half_x) {
       const float il = lsum > 0.f ? 1.f / lsum : 0.f;

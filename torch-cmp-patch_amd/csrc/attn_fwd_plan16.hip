@@ -82,13 +82,22 @@ int exchange_waves(int n_qblk, int Sq) {
   return n_qblk > 1 ? kPipeNw : (Sq + 31) / 32 < kPipeNw ? (Sq + 31) / 32 : kPipeNw;
 }
 
-// What the plan weighs besides the grid: the head-dim bucket, whether two
-// parts exchange O in 16 bits (fp16), and whether the block is short (decode,
-// packed rows: at most 64 rows, a launch bound by the K/V stream).
+// What the plan weighs besides the grid: the head-dim bucket, the element type,
+// and whether the block is short (decode, packed rows: at most 64 rows, a
+// launch bound by the K/V stream).
 struct PlanKind {
   int dk;
-  bool half, shortq;
+  bool f16, shortq;
 };
+
+// Whether two parts exchange O / l in fp16: fp16 launches whose grid and sweep
+// allow two parts and no more (SDXL self-attention).  Where more would fit and
+// the plan takes two because they are faster, as where fewer would, the
+// exchange is fp32, as that of three and more: a second fp16 rounding of O
+// would make the result less exact than the finer cut it replaces (rms
+// error against 64 bits, N(0,1) inputs, [1,12,1024,1024,64]: 1.15 times the
+// unsplit one with the fp16 exchange, 1.00 with fp32).
+bool half_exchange(const PlanKind& k, int most) { return k.f16 && most == 2; }
 
 // Cost of cutting a block's sweep in two, in key tiles of one block: the
 // prologue, the exchange and the merge of one block (about 3 us) and each
@@ -97,27 +106,27 @@ struct PlanKind {
 // 3072): where it exceeds the tiles a cut saves, the cut launch was the slower
 // one, by up to half (bf16 [1,32,1024,1024,128], 256 blocks: 24 us whole, 37
 // us cut), and with few exceptions only there.
-float cut_cost(const PlanKind& k, int n) {
-  const float per_block = k.dk > 128 ? 0.057f : k.dk > 64 ? (k.half ? 0.063f : 0.114f) : (k.half ? 0.034f : 0.063f);
-  const float base = !k.half || k.dk > 128 ? 6.f : k.dk > 64 ? 7.f : 8.f;
+float cut_cost(int dk, bool half, int n) {
+  const float per_block = dk > 128 ? 0.057f : dk > 64 ? (half ? 0.063f : 0.114f) : (half ? 0.034f : 0.063f);
+  const float base = !half || dk > 128 ? 6.f : dk > 64 ? 7.f : 8.f;
   return base + per_block * n;
 }
 
-// Parts of every block of a non-causal prefill with fewer blocks than CUs.
+// Parts of every block of a non-causal prefill with fewer blocks than CUs
+// (half: two of them exchange in fp16).
 // With a part to a CU, P parts save nt (1 - 1/P) tiles; two parts beyond that
 // share CUs and save 0.38 nt (above D = 128 a CU holds one workgroup: nothing).  Three parts and more all leave fp32 states, and
 // from four on a launch pays another 5 (D > 128) or 12 tiles: bf16
 // [1,8,1024,1024,D], 64 blocks, whole / in 2 / 3 / 4 parts, D = 64: 16.1 / 13.8
 // / 12.8 / 17.2 us, D = 128: 21.5 / 19.9 / 19.4 / 23.1, D = 256: 46.7 / 37.5 /
 // 34.3 / 37.1.
-int prefill_parts(const PlanKind& k, int n, int nt, int cus, int occ) {
-  const float save2 = nt * (2 * n <= cus ? 0.5f : occ > 1 ? 0.38f : 0.f) - cut_cost(k, n);
+int prefill_parts(int dk, bool half, int n, int nt, int cus, int occ) {
+  const float save2 = nt * (2 * n <= cus ? 0.5f : occ > 1 ? 0.38f : 0.f) - cut_cost(dk, half, n);
   int parts = save2 > 0.f ? 2 : 1;
   float best = save2 > 0.f ? save2 : 0.f;
-  const PlanKind full = {k.dk, false, false};
   for (int p = 3; p <= nt / kMinPartTiles && n * p <= cus; ++p) {
-    const float many = p > 3 ? (k.dk > 128 ? 5.f : 12.f) : k.dk > 64 && k.dk <= 128 ? 2.f : 0.f;
-    const float save = nt * (1.f - 1.f / p) - cut_cost(full, n * p / 2) - many;
+    const float many = p > 3 ? (dk > 128 ? 5.f : 12.f) : dk > 64 && dk <= 128 ? 2.f : 0.f;
+    const float save = nt * (1.f - 1.f / p) - cut_cost(dk, false, n * p / 2) - many;
     if (save > best) {
       best = save;
       parts = p;
@@ -156,44 +165,44 @@ SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntile
   if (causal) {
     const int slots = occ * cus;
     if (n * 2 > slots || (n * 2 > cus && ntiles < kLongCausalTiles)) return sa;
-    int parts = slots / n;
-    if (parts > ntiles / kMinCausalPartTiles) parts = ntiles / kMinCausalPartTiles;
+    int most = slots / n;
+    if (most > ntiles / kMinCausalPartTiles) most = ntiles / kMinCausalPartTiles;
+    if (most > ntiles_min) most = ntiles_min;
+    if (most > kMaxCausalParts) most = kMaxCausalParts;
+    int parts = most;
     if (parts > 2 && parts > ntiles / kMinManyCausalTiles)
       parts = ntiles / kMinManyCausalTiles > 2 ? ntiles / kMinManyCausalTiles : 2;
     if (parts > 3 && n * 3 > cus) parts = 3;
-    if (parts > ntiles_min) parts = ntiles_min;
-    if (parts > kMaxCausalParts) parts = kMaxCausalParts;
     if (parts < 2) return sa;
     sa.nfull = 0;
     sa.nparts = parts;
+    sa.half16 = half_exchange(k, most);
     return sa;
   }
   const int full = n / cus, rem = n - full * cus;
   if (rem == 0 || full + 1 > occ) return sa;  // whole rounds, or more than fits at once
-  int parts;
+  // After whole rounds each CU takes at most one part of the round that
+  // remains.  With no whole round each CU can hold several parts at once: more
+  // key ranges streamed side by side, more loads in flight (a decode step with
+  // one part per CU reaches ~5.2 TB/s).
+  const int per_cu = full == 0 ? (occ < kMaxPartsPerCu ? occ : kMaxPartsPerCu) : 1;
+  int most = per_cu * cus / rem;
+  if (most > ntiles / kMinPartTiles) most = ntiles / kMinPartTiles;
+  int parts = most;
   if (full == 0 && !k.shortq) {
-    parts = prefill_parts(k, n, ntiles, cus, occ);
-  } else {
-    // After whole rounds each CU takes at most one part of the round that
-    // remains.  With no whole round of short blocks (decode, short sweeps) each
-    // CU can hold several parts at once: more key ranges streamed side by side,
-    // more loads in flight (a decode step with one part per CU reaches ~5.2
-    // TB/s).
-    const int per_cu = full == 0 ? (occ < kMaxPartsPerCu ? occ : kMaxPartsPerCu) : 1;
-    parts = per_cu * cus / rem;
-    if (parts > ntiles / kMinPartTiles) parts = ntiles / kMinPartTiles;
-    if (full > 0 && !k.shortq) {
-      // the tail of a prefill: two parts (bf16 [1,20,2048,2048,64], 64 blocks
-      // left: whole 35.8 us, 2 parts 31.8, 3 32.2, 4 33.9), and where each CU
-      // would take little less than a whole block more, only of long sweeps
-      // ([1,64,768,768,64], 128 left: 17.9 whole, 18.2 cut; 1536: 29.8, 28.1)
-      if (parts > 2) parts = 2;
-      if (rem * 2 >= cus && ntiles < kMinTailTiles) parts = 1;
-    }
+    parts = prefill_parts(k.dk, k.f16 && most <= 2, n, ntiles, cus, occ);
+  } else if (full > 0 && !k.shortq) {
+    // the tail of a prefill: two parts (bf16 [1,20,2048,2048,64], 64 blocks
+    // left: whole 35.8 us, 2 parts 31.8, 3 32.2, 4 33.9), and where each CU
+    // would take little less than a whole block more, only of long sweeps
+    // ([1,64,768,768,64], 128 left: 17.9 whole, 18.2 cut; 1536: 29.8, 28.1)
+    if (parts > 2) parts = 2;
+    if (rem * 2 >= cus && ntiles < kMinTailTiles) parts = 1;
   }
   if (parts < 2) return sa;
   sa.nfull = full * cus;
   sa.nparts = parts;
+  sa.half16 = half_exchange(k, most);
   return sa;
 }
 
