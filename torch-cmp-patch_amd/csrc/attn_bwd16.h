@@ -223,6 +223,41 @@ __device__ __forceinline__ float mask_elem(__amdgpu_buffer_rsrc_t rs, int off, i
   return f * kLog2e;
 }
 
+// The same of 16 rows of one key column, register r's row acc_key(r, 0) rows of
+// `step` bytes past `off`.  The kind is looked at once and BATCH loads go out
+// together: tested per element, each load stood in a branch of its own that
+// waited for it and for the next tile's loads before it, 16 times a tile (whole
+// backward, a mask row per query: bf16 causal [2,16/8,2048,2048,256] 938 -> 518
+// us, [4,16/8,2048,2048,64] 523 -> 238, fp16 [2,10,4096,4096,64] 902 -> 488).
+template <int BATCH>
+__device__ __forceinline__ void mask_elems16(__amdgpu_buffer_rsrc_t rs, uint32_t off, uint32_t step, int kind,
+                                             float (&a)[16]) {
+  auto all = [&](auto load, auto value) {
+#pragma unroll
+    for (int r0 = 0; r0 < 16; r0 += BATCH) {
+      uint32_t w[BATCH];
+#pragma unroll
+      for (int r = 0; r < BATCH; ++r) w[r] = load((int)(off + acc_key(r0 + r, 0) * step));
+#pragma unroll
+      for (int r = 0; r < BATCH; ++r) a[r0 + r] = value(w[r]);
+      if (BATCH < 16) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (kind == MASK_BOOL)
+    all([&](int o) -> uint32_t { return __builtin_amdgcn_raw_buffer_load_b8(rs, o, 0, 0); },
+        [](uint32_t w) { return w ? 0.f : -INFINITY; });
+  else if (kind == MASK_F32)
+    all([&](int o) -> uint32_t { return __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0); },
+        [](uint32_t w) { return __uint_as_float(w) * kLog2e; });
+  else
+    all([&](int o) -> uint32_t { return __builtin_amdgcn_raw_buffer_load_b16(rs, o, 0, 0); },
+        [&](uint32_t w) {
+          const float f = kind == MASK_F16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)w)
+                                           : __uint_as_float(w << 16);
+          return f * kLog2e;
+        });
+}
+
 // ---- Delta_i = sum_d dO_id * O_id (fp32), 8 lanes per row
 template <typename T>
 __global__ void __launch_bounds__(256) attn_bwd_delta(const BwdParams p) {
@@ -378,6 +413,11 @@ struct BwdDkdv {
                             : DK == 128 ? (MASK != CAUSAL ? 2 : 0)
                             : DK == 256 ? (MASK && CAUSAL ? 3 : 0)
                                         : 0;
+  // mask loads of a tile in flight at once, where each query row has its own:
+  // all 16, or 8 where 16 more registers are not to be had (up to D = 128 not
+  // causal: with 16 the sweep spills, and key masks pay for it too: bf16
+  // [2,16/8,2048,2048,128] 289 us with 8, 293 with 16)
+  static constexpr int MBATCH = DK <= 128 && !CAUSAL ? 8 : 16;
   // halves: an operand is 16 bytes per thread, at consecutive addresses (no
   // bank conflicts, no padding)
   static constexpr int PARK = ((VLDS ? DK / 16 : 0) + KP) * 256 * 8 + (VLDS || KP > 0 ? 0 : 8);
@@ -592,9 +632,8 @@ __device__ __forceinline__ void bwd_dkdv_block(const BwdParams& p, const int wg,
 #pragma unroll
           for (int r = 0; r < 16; ++r) madd[r] = a;
         } else {
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            madd[r] = mask_elem(mrs, (int)(((int64_t)(q0 + acc_key(r, hh)) * p.m_q + key) * mes), kind);
+          mask_elems16<Cfg::MBATCH>(mrs, (uint32_t)(((int64_t)(q0 + 8 * hh) * p.m_q + key) * mes),
+                                    (uint32_t)(p.m_q * mes), kind, madd);
         }
       }
       // register r holds query q0 + acc_key(r, hh): two runs of 8 consecutive rows
