@@ -101,3 +101,17 @@ print(json.dumps([sorted(rcs), launches()]))
     assert len(bits) == (16 if other == "masked" else 8)
     for i in bits:
         assert seen[i + 1][0] == seen[i][0] and "attn_fwd_pipe16" in seen[i + 1][1], seen[max(0, i - 2):i + 4]
+
+
+# HIP takes fewer than 2^32 threads per grid.  Many short sequences: each
+# gradient sweep's grid is within that, the two together are not.
+@pytest.mark.parametrize("dt,D,causal", [("F16", 64, 0), ("BF16", 64, 1), ("BF16", 128, 0), ("F32", 32, 1), ("F32", 40, 0)])
+def test_backward_grids_stay_launchable(recorder, dt, D, causal):
+    rc, seen = _run(recorder, f"""
+rc = bwd({dt}, 3000, 3000, 3000, 1, 1, {D}, {causal})
+print(json.dumps([rc, launches()]))
+""")
+    assert rc == 0
+    assert all(threads < 2 ** 32 for *_, threads in seen), seen
+    # nothing is lost: a workgroup per block of keys and of queries
+    assert sum(wg for _, name, wg, _ in seen if "grads" in name) == 2 * 3000 * 3000

@@ -1090,4 +1090,19 @@ attn_bwd_grads(const BwdParams p) {
     bwd_dq_block<T, DK, CAUSAL, MASK>(p, SWEEP == BWD_BOTH ? wg - p.n_wg : wg, lds, park);
 }
 
+// Launch both sweeps: one grid, or one each where the two together are more
+// threads than a grid may have (2^32; many short sequences).
+constexpr int64_t kMaxGridWgs = (int64_t(1) << 32) / 256 - 1;
+template <typename K>
+void launch_both_sweeps(K kernel, const BwdParams& p, hipStream_t s) {
+  if ((int64_t)p.n_wg + p.n_wg_q <= kMaxGridWgs) {
+    hipLaunchKernelGGL(kernel, dim3(p.n_wg + p.n_wg_q), dim3(256), 0, s, p);
+    return;
+  }
+  hipLaunchKernelGGL(kernel, dim3(p.n_wg), dim3(256), 0, s, p);
+  BwdParams q = p;
+  q.n_wg = 0;  // every workgroup is a dQ one
+  hipLaunchKernelGGL(kernel, dim3(q.n_wg_q), dim3(256), 0, s, q);
+}
+
 }  // namespace cmpext3

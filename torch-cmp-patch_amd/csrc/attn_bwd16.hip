@@ -34,8 +34,7 @@ hipError_t launch_bwd_t(const BwdParams& p0, hipStream_t s) {
       hipLaunchKernelGGL((attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_DQ>), dim3(p.n_wg_q), dim3(256), 0, s, p);
     }
   }
-  if (!apart)
-    hipLaunchKernelGGL((attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_BOTH>), dim3(p.n_wg + p.n_wg_q), dim3(256), 0, s, p);
+  if (!apart) launch_both_sweeps(attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_BOTH>, p, s);
   if (p.nfull > 0) {
     const int64_t n4 = (int64_t)(n_kv - p.nfull) * 128 * p.D / 4;
     hipLaunchKernelGGL((attn_bwd_tail_sum<T, true>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, p);

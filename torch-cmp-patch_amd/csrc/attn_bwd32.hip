@@ -543,8 +543,7 @@ hipError_t launch_bwd32_t(const BwdParams& p0, hipStream_t s) {
       hipLaunchKernelGGL((attn_bwd32_grads<DK, CAUSAL, BWD_DQ>), dim3(p.n_wg_q), dim3(256), 0, s, p);
     }
   }
-  if (!apart)
-    hipLaunchKernelGGL((attn_bwd32_grads<DK, CAUSAL, BWD_BOTH>), dim3(p.n_wg + p.n_wg_q), dim3(256), 0, s, p);
+  if (!apart) launch_both_sweeps(attn_bwd32_grads<DK, CAUSAL, BWD_BOTH>, p, s);
   launch_part_sums<float>(p, ns > 1, nsq > 1, s);
   return hipGetLastError();
 }
