@@ -92,7 +92,12 @@ struct BwdParams {
 // rounds).  A causal launch does half the work; while its workgroups are all
 // resident the longest sets its time.  Least squares over 371 backward calls on
 // MI355X (8 to 64 heads, 100 to 3072 tokens, f16/bf16 D = 64, 128, 256 and fp32
-// D = 40, 64, 128, each whole and in up to two plans).
+// D = 40, 64, 128, each whole and in up to two plans), measured with a launch per
+// sweep.  It knows nothing of the other sweep, whose workgroups share the one
+// launch: over 1010 f16/bf16 and 460 fp32 calls timed there with every pair of
+// parts, the pair that the two sweeps' plans give is 5% (fp32 4%) slower than
+// the best pair on average, up to a third where the other sweep already fills
+// the chip (bf16 causal [2,32/16,2039,2039,128] 301 us, whole 258).
 inline float sweep_us(int64_t n_wg, int ns, int occ, int cus, bool causal, int64_t tiles, float tile_us,
                       float part_mb) {
   float k = (float)(n_wg * ns) / cus;
@@ -159,16 +164,18 @@ struct BwdSplit {
 };
 
 // Split tail of a non-causal grid of n equal sweeps that fills more than one
-// but not a whole number of rounds of one workgroup per CU, within the occ
-// workgroups per CU the kernel allows (SDXL self-attention: 640 blocks at
-// three per CU): the blocks past the whole rounds are cut into parts, one
-// per CU, so every CU holds the same work (as the forward's key split does).
+// but not a whole number of rounds of one workgroup per CU, the partial round
+// being the last that the occ workgroups a CU holds leave room for (SDXL
+// self-attention: 640 blocks at three per CU): the blocks past the whole rounds
+// are cut into parts, one per CU, so every CU holds the same work (as the
+// forward's key split does).  A partial round before the last is filled by the
+// other sweep's workgroups.
 // Returns the parts (1 = none) and sets *nfull.
 inline int split_tail(int64_t n, int occ, int cus, int64_t tiles, int* nfull) {
   *nfull = 0;
   if (cus <= 0) return 1;
   const int64_t full = n / cus, rem = n - full * cus;
-  if (full == 0 || rem == 0 || full + 1 > occ) return 1;
+  if (full == 0 || rem == 0 || full + 1 != occ) return 1;
   int64_t ns = cus / rem;
   if (ns > 8) ns = 8;
   if (ns > tiles / 8) ns = tiles / 8;

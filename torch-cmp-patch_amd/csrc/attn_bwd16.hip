@@ -66,30 +66,38 @@ hipError_t launch_bwd_dtype(const BwdParams& p, int dk, bool causal, hipStream_t
 
 int bwd16_bucket(int D) { return D <= 0 ? -1 : D <= 64 ? 64 : D <= 128 ? 128 : D <= 192 ? 192 : D <= 256 ? 256 : -1; }
 
+// Workgroups of the one launch that a CU holds.
+template <int DK>
+static int grads_occ(bool causal, bool masked) {
+  if (masked) return causal ? bwd_occ<DK, true, true, BWD_BOTH>() : bwd_occ<DK, false, true, BWD_BOTH>();
+  return causal ? bwd_occ<DK, true, false, BWD_BOTH>() : bwd_occ<DK, false, false, BWD_BOTH>();
+}
+
 // Split plan of the f16/bf16 gradient sweeps (split_sweep): dK/dV over
 // 128-key blocks, each sweeping (query head of the group, 32-query tile);
-// dQ over 128-query blocks, each sweeping 32-key tiles.  Workgroups per CU
-// follow the kernels' waves per SIMD.
+// dQ over 128-query blocks, each sweeping 32-key tiles.
 BwdSplit bwd16_split(int B, int H, int Hkv, int Sq, int Sk, int D, bool causal, bool masked, int cus) {
   BwdSplit sp;
   const int dk = bwd16_bucket(D);
   if (dk < 0 || (int64_t)B * H * Sq == 0 || Hkv < 1) return sp;
-  const int occ_kv = dk <= 64 ? (causal ? 2 : 3) : dk <= 128 ? (masked && causal ? 1 : 2) : 1;
-  const int occ_q = dk <= 64 ? (masked ? 2 : 3) : dk <= 128 ? (masked && causal ? 1 : 2) : 1;
+  const int occ = dk == 64    ? grads_occ<64>(causal, masked)
+                  : dk == 128 ? grads_occ<128>(causal, masked)
+                  : dk == 192 ? grads_occ<192>(causal, masked)
+                              : grads_occ<256>(causal, masked);
   const int64_t n_kv = (int64_t)B * Hkv * ((Sk + 127) / 128), n_q = (int64_t)B * H * ((Sq + 127) / 128);
   const int64_t t_kv = (int64_t)(H / Hkv) * ((Sq + 31) / 32), t_q = (Sk + 31) / 32;
-  // us per 32-row tile of one block, a CU to itself.  Masked tiles take 1.2 (a
-  // mask for all query rows) to 2.3 times (a row each) as long: weighed 1 and
-  // 1.7, D = 64 backwards gain 1.24 and 1.21 times over the most parts with key
-  // masks, 1.11 and 1.24 with a row each (geometric means of 17 shapes)
-  const float mx = masked ? 1.7f : 1.f;
-  const float us_kv = dk <= 64 ? 0.74f : dk <= 128 ? 1.2f : dk <= 192 ? 2.f : 2.8f;
-  const float us_q = dk <= 64 ? 0.49f : dk <= 128 ? 0.86f : dk <= 192 ? 1.35f : 1.83f;
-  sp.ns_kv = split_sweep(n_kv, occ_kv, cus, causal, t_kv, mx * us_kv, 8e-6f * B * Hkv * Sk * D);
-  sp.ns_q = split_sweep(n_q, occ_q, cus, causal, t_q, mx * us_q, 4e-6f * B * H * Sq * D);
+  // us per 32-row tile of one block, a CU to itself.  A mask costs dQ tiles more
+  // than dK/dV ones (260 calls that both weighed 1.7, the dQ sweep of masked D <=
+  // 64 at two workgroups per CU and a tail in any round planned otherwise: 7%
+  // faster on average, 186 by over 3%, six slower by over 3%; dK/dV weighed 1, 22
+  // slower by over 3%, some short grids of few heads by up to 20%)
+  const float us_kv = (masked ? 1.25f : 1.f) * (dk <= 64 ? 0.74f : dk <= 128 ? 1.2f : dk <= 192 ? 2.f : 2.8f);
+  const float us_q = (masked ? 1.7f : 1.f) * (dk <= 64 ? 0.49f : dk <= 128 ? 0.86f : dk <= 192 ? 1.35f : 1.83f);
+  sp.ns_kv = split_sweep(n_kv, occ, cus, causal, t_kv, us_kv, 8e-6f * B * Hkv * Sk * D);
+  sp.ns_q = split_sweep(n_q, occ, cus, causal, t_q, us_q, 4e-6f * B * H * Sq * D);
   // non-causal grids past one round: split only the last, partial round
-  if (!causal && sp.ns_kv == 1) sp.ns_kv = split_tail(n_kv, occ_kv, cus, t_kv, &sp.nfull_kv);
-  if (!causal && sp.ns_q == 1) sp.ns_q = split_tail(n_q, occ_q, cus, t_q, &sp.nfull_q);
+  if (!causal && sp.ns_kv == 1) sp.ns_kv = split_tail(n_kv, occ, cus, t_kv, &sp.nfull_kv);
+  if (!causal && sp.ns_q == 1) sp.ns_q = split_tail(n_q, occ, cus, t_q, &sp.nfull_q);
   return sp;
 }
 

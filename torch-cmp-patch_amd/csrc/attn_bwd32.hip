@@ -572,9 +572,11 @@ int bwd32_bucket(int D) {
 
 // Split plan of the fp32 gradient sweeps (split_sweep): dK/dV over 64-key
 // blocks sweeping 32-query tiles, dQ over 64-query blocks sweeping 32-key
-// tiles.  Workgroups per CU from the kernels' registers and LDS: dK/dV 5 at
-// D <= 32, 4 up to 40, 3 (causal 4) up to 64, 2 up to 128, then 1; dQ 7, 5,
-// 4, 3 up to 96, 2 up to 128, then 1.
+// tiles.  Workgroups per CU from the registers and LDS of each sweep by itself:
+// dK/dV 5 at D <= 32, 4 up to 40, 3 (causal 4) up to 64, 2 up to 128, then 1;
+// dQ 7, 5, 4, 3 up to 96, 2 up to 128, then 1 (beside dK/dV in the one launch it
+// has dK/dV's; the finer cut that its own count gives is kept, as the parts
+// fill the tail of the dK/dV ones).
 BwdSplit bwd32_split(int B, int H, int Hkv, int Sq, int Sk, int D, bool causal, int cus) {
   BwdSplit sp;
   const int dk = bwd32_bucket(D);
