@@ -186,12 +186,17 @@ inline int split_tail(int64_t n, int occ, int cus, int64_t tiles, int* nfull) {
 
 // Whether a dK/dV grid of n blocks leaves (almost) none of its last
 // round of `slots` empty.  Where the dQ sweep runs a wave per SIMD more by itself
-// than beside the dK/dV sweep, such a grid takes its own launch: there is no
-// tail for the dQ workgroups to fill (same MI355X run, in one launch and in two:
-// bf16 causal with a key mask [4,16/8,2048,2048,64] 208 and 199 us; fp32
-// [2,8,3000,3000,40] 812 and 775, causal [2,8,3000,3000,32] 343 and 326; kernels
-// without that wave gain up to 8% from one launch there too, as at bf16 causal
-// [4,16/8,1024,1024,256] 249 and 270).
+// than beside the dK/dV sweep, such a grid may take its own launch: there is no
+// tail for the dQ workgroups to fill.  16-bit masked causal D <= 64 does where the
+// dQ grid is two rounds or more and the dK/dV grid is too, or the sweeps are long
+// (same MI355X run, in one launch and in two: bf16 key mask
+// [4,16/8,2048,2048,64] 206 and 199 us, [2,32/16,4096,4096,64] 643 and 616; with 512
+// dQ blocks [2,16,2048,2048,64] 111 and 131, and with 512 dK/dV blocks of 1024 rows
+// [4,32/16,1024,1024,64] 132 and 154), unmasked causal does not
+// ([4,16/8,2048,2048,64] 166 and 172); fp32 D <= 40 does ([2,8,3000,3000,40]
+// 815 and 775, causal [2,8,3000,3000,32] 343 and 325).  Kernels without that wave
+// gain up to 8% from one launch there too, as at bf16 causal
+// [4,16/8,1024,1024,256] 249 and 270.
 inline bool last_round_full(int64_t n, int64_t slots) {
   return n >= slots && (n + slots - 1) / slots * slots - n <= slots / 10;
 }
@@ -827,7 +832,7 @@ template <int DK, bool CAUSAL, bool MASK>
 struct BwdDq {
   static constexpr int BQ = 128, BK = 32;
   static constexpr int RS = bwd_lds_stride(DK);
-  static constexpr int OCC = DK <= 64 ? (MASK && CAUSAL ? 2 : 3) : (DK > 128 || (MASK && CAUSAL)) ? 1 : 2;
+  static constexpr int OCC = DK <= 64 ? 3 : (DK > 128 || (MASK && CAUSAL)) ? 1 : 2;
   // D > 64 masked non-causal: the dO operands live in LDS (each lane reads
   // back only what it wrote; no barrier), which leaves room for 2 waves per
   // SIMD instead of 1 (masked backward 473 -> 419 us on bf16

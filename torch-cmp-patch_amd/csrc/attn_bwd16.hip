@@ -27,8 +27,9 @@ hipError_t launch_bwd_t(const BwdParams& p0, hipStream_t s) {
   const int n_q = p.B * p.H * p.n_blk_q;
   p.n_wg_q = p.nfull_q > 0 ? p.nfull_q + (n_q - p.nfull_q) * nsq : n_q * nsq;
   bool apart = false;
-  if constexpr (DK == 64 && CAUSAL) {
-    apart = last_round_full(n_kv, (int64_t)BwdDkdv<DK, CAUSAL, MASK>::OCC * device_cus());
+  if constexpr (DK == 64 && CAUSAL && MASK) {
+    const int64_t slots = (int64_t)BwdDkdv<DK, CAUSAL, MASK>::OCC * device_cus();
+    apart = last_round_full(n_kv, slots) && n_q >= 2 * slots && (n_kv >= 2 * slots || p.Sk >= 1792);
     if (apart) {
       hipLaunchKernelGGL((attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_DKDV>), dim3(p.n_wg), dim3(256), 0, s, p);
       hipLaunchKernelGGL((attn_bwd_grads<T, DK, CAUSAL, MASK, BWD_DQ>), dim3(p.n_wg_q), dim3(256), 0, s, p);
