@@ -42,9 +42,11 @@ def _reference(q, k, v, do, scale, causal, mask):
 
 
 @pytest.mark.parametrize("dtype,B,H,Hkv,S,D,causal,masked", [
-    (BF16, 2, 16, 16, 2048, 64, True, False),   # 512 key blocks, two a CU: a launch each
+    (BF16, 2, 16, 16, 2048, 64, True, False),   # 512 key blocks, two a CU
     (F16, 2, 16, 16, 2047, 64, True, True),
-    (BF16, 2, 15, 15, 2048, 64, True, False),   # 480: one launch
+    (F16, 2, 32, 16, 2047, 64, True, True),     # and 1024 query blocks, masked: a launch each
+    (BF16, 4, 16, 16, 1000, 64, True, True),    # 512 and 512: one launch
+    (BF16, 2, 15, 15, 2048, 64, True, False),
     (F16, 2, 6, 3, 333, 64, False, True),       # K operands parked
     (F32, 2, 8, 8, 2040, 40, False, False),     # 512 key blocks: a launch each
     (F32, 2, 8, 8, 1890, 40, False, False),     # 480: one launch

@@ -37,10 +37,10 @@ def fwd(entry, dt, B, H, S, D, mask, ws=None, nbytes=0, causal=0):
         tail += [None]
         f = lib.cmpext3_attn_fwd_noalloc
     return f(vp(A), vp(A), vp(A), vp(A), dt, B, H, H, S, S, D, st, st, st, st, *tail)
-def bwd(dt, B, H, Hkv, Sq, Sk, D, causal, ws=None, nbytes=0):
+def bwd(dt, B, H, Hkv, Sq, Sk, D, causal, ws=None, nbytes=0, mask=False):
     q, k = s3(H * Sq * D, Sq * D, D), s3(Hkv * Sk * D, Sk * D, D)
-    return lib.cmpext3_attn_bwd_ws(*[vp(A)] * 10, dt, B, H, Hkv, Sq, Sk, D, q, k, k, q, q, q, k, k, None, -1,
-                                   s3(0, 0, 0), ctypes.c_float(0.1), causal, vp(ws), sz(nbytes), None)
+    return lib.cmpext3_attn_bwd_ws(*[vp(A)] * 10, dt, B, H, Hkv, Sq, Sk, D, q, k, k, q, q, q, k, k,
+                                   vp(A) if mask else None, BOOL if mask else -1, s3(0, 0, 0), ctypes.c_float(0.1), causal, vp(ws), sz(nbytes), None)
 def launches():
     out = []
     for i in range(rec.recorder_count()):
@@ -115,3 +115,38 @@ print(json.dumps([rc, launches()]))
     assert all(threads < 2 ** 32 for *_, threads in seen), seen
     # nothing is lost: a workgroup per block of keys and of queries
     assert sum(wg for _, name, wg, _ in seen if "grads" in name) == 2 * 3000 * 3000
+
+
+# The gradient sweeps share one launch, except where the dQ sweep runs a wave
+# per SIMD more by itself and both grids fill their rounds.
+@pytest.mark.parametrize("dt,B,H,Hkv,S,D,causal,mask,n", [
+    ("BF16", 4, 16, 8, 2048, 64, 1, True, 2),
+    ("BF16", 4, 32, 32, 1024, 64, 1, True, 2),
+    ("BF16", 4, 16, 8, 2048, 64, 1, False, 1),     # without a mask
+    ("BF16", 2, 16, 16, 2048, 64, 1, True, 1),     # 512 dQ blocks
+    ("BF16", 4, 32, 16, 1024, 64, 1, True, 1),     # 512 dK/dV blocks of short sweeps
+    ("BF16", 4, 15, 15, 2048, 64, 1, True, 1),     # a partial round
+    ("F16", 4, 32, 32, 1024, 64, 0, True, 1),
+    ("F32", 2, 8, 8, 3000, 40, 0, False, 2),
+    ("F32", 2, 8, 8, 3000, 64, 0, False, 1),
+])
+def test_backward_launch_forms(recorder, dt, B, H, Hkv, S, D, causal, mask, n):
+    rc, seen = _run(recorder, f"""
+rc = bwd({dt}, {B}, {H}, {Hkv}, {S}, {S}, {D}, {causal}, mask={mask})
+print(json.dumps([rc, launches()]))
+""")
+    assert rc == 0
+    assert sum("grads" in name for _, name, *_ in seen) == n
+
+
+def test_backward_plans_count_the_one_launch():
+    """Three workgroups per CU at D <= 64, masked too (a dQ grid of 128 blocks
+    takes six parts); a partial round is cut only where it is the last that
+    the CUs have room for (no tails of 384 blocks at three per CU)."""
+    import torch
+    from cmpext3 import abi
+    if torch.cuda.is_available():
+        pytest.skip("plan depends on the visible device's CU count")
+    size = lambda B, H, S, mask: abi.bwd_workspace_size(abi.DTYPE_F16, B, H, H, S, S, 64, mask, False)
+    assert size(1, 8, 2048, abi.DTYPE_BOOL) == (2 * 6 + 6) * 8 * 2048 * 64 * 4
+    assert size(4, 16, 700, -1) == 0
