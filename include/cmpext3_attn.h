@@ -209,7 +209,7 @@ size_t cmpext3_attn_fwd_workspace_size(int dtype, int B, int H, int H_kv, int Sq
  * launch then loads no mask elements and leaves out the key tiles a query
  * block keeps no key of.  One bit per mask element (dimensions of stride 0
  * once) and a byte per 128 rows x 32 keys.  0 when the launch has no use for
- * it.  With less workspace the mask is read as it is: the same result within
+ * it, whatever the alignment of the mask's base and of the tensors.  With less workspace the mask is read as it is: the same result within
  * rounding.  Host-only.
  */
 size_t cmpext3_attn_fwd_mask_workspace_size(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D,

@@ -150,3 +150,26 @@ def test_backward_plans_count_the_one_launch():
     size = lambda B, H, S, mask: abi.bwd_workspace_size(abi.DTYPE_F16, B, H, H, S, S, 64, mask, False)
     assert size(1, 8, 2048, abi.DTYPE_BOOL) == (2 * 6 + 6) * 8 * 2048 * 64 * 4
     assert size(4, 16, 700, -1) == 0
+
+
+def test_mask_workspace_is_asked_for_by_launches_that_fill_it(recorder):
+    """The size query against the launches: bytes exactly where a call with room
+    for them makes the bits (element-wise masks: Sk not a multiple of 8)."""
+    got = _run(recorder, """
+lib.cmpext3_attn_fwd_mask_workspace_size.restype = sz
+out = []
+for dt in (F16, BF16, F32):
+    for B, H, S in ((1, 4, 1), (2, 4, 20), (2, 4, 77), (4, 16, 203), (1, 8, 517), (2, 8, 2045)):
+        for D in (32, 44, 64, 80, 100, 128, 160, 192, 256):
+            for causal in (0, 1):
+                rec.recorder_clear()
+                size = lib.cmpext3_attn_fwd_mask_workspace_size(dt, B, H, H, S, S, D, BOOL, s3(0, 0, S), causal)
+                if dt == F32 and D % 4:
+                    continue
+                rc = fwd("ws", dt, B, H, S, D, True, 1 << 34, 1 << 30, causal)
+                out.append([dt, B, H, S, D, causal, rc, size, sum("attn_mask_bits" in n for _, n, *_ in launches())])
+print(json.dumps(out))
+""")
+    assert len(got) > 300 and any(size for *_, size, _ in got)
+    for *case, rc, size, made in got:
+        assert rc == 0 and (size > 0) == (made == 1), (case, size, made)

@@ -31,7 +31,6 @@ BwdSplit bwd_split(int dtype, int B, int H, int Hkv, int Sq, int Sk, int D, bool
 hipError_t launch_bwd32(const BwdParams& p, bool causal, hipStream_t s);
 hipError_t launch_mfma16(const FwdParams& p, bool bf16, bool causal, hipStream_t s);
 hipError_t launch_mfma32(const FwdParams& p, bool causal, hipStream_t s);
-bool decode16_applies(const FwdParams& p, bool causal);
 int mfma16_bucket(int D);
 int mfma32_bucket(int D);
 void describe_mfma16(int D, int B, int H, int Sq, int Sk, bool causal, bool bf16, char* buf, int len);
@@ -307,10 +306,11 @@ int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, i
 // plan recorded is the one a launch would take with workspace_bytes of
 // workspace.  Touches no device (the CU count falls back to MI355X's 256
 // when none is visible).
+// mask_str (may be null): the mask's strides, its rows read element by element.
 int plan_impl(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D, int mask_dtype, int causal,
-              int with_lse, int elem, size_t workspace_bytes, cmpext3::SplitInfo& info) {
-  info.need = 0;
-  info.parts = 1;
+              int with_lse, int elem, size_t workspace_bytes, cmpext3::SplitInfo& info,
+              const int64_t* mask_str = nullptr) {
+  info = cmpext3::SplitInfo{0, 1};
   int rc = check_shape(dtype, B, H, Sq, Sk, D);
   if (rc != CMPEXT3_OK || (int64_t)B * H * Sq == 0) return rc;
   if (H_kv < 1 || H_kv > H || H % H_kv != 0) return CMPEXT3_E_INVALID;
@@ -329,6 +329,10 @@ int plan_impl(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D, int mask
   p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.D = D;
   p.kv_group = H / H_kv;
   p.mask_kind = mask_dtype == -1 ? cmpext3::MASK_NONE : mask_kind_of(mask_dtype);
+  if (mask_str) {
+    p.m_b = mask_str[0]; p.m_h = mask_str[1]; p.m_q = mask_str[2];
+    p.mask_narrow = 1;
+  }
   p.lse = with_lse ? (float*)&info : nullptr;  // never dereferenced: marks the training forward
   p.c = 0.125f;
   p.workspace_bytes = workspace_bytes;
@@ -363,22 +367,16 @@ size_t cmpext3_attn_fwd_workspace_size(int dtype, int B, int H, int H_kv, int Sq
 
 size_t cmpext3_attn_fwd_mask_workspace_size(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D,
                                             int mask_dtype, const int64_t mask_str[3], int causal) {
-  if (check_shape(dtype, B, H, Sq, Sk, D) != CMPEXT3_OK || (int64_t)B * H * Sq == 0) return 0;
-  if (dtype == CMPEXT3_DTYPE_F32 || mask_dtype != CMPEXT3_DTYPE_BOOL || !mask_str) return 0;
-  if (H_kv < 1 || H_kv > H || H % H_kv != 0) return 0;
-  cmpext3::FwdParams p;
-  memset(&p, 0, sizeof p);
-  p.B = B; p.H = H; p.Sq = Sq; p.Sk = Sk; p.D = D;
-  p.kv_group = H / H_kv;
-  p.mask_kind = cmpext3::MASK_BOOL;
-  p.m_b = mask_str[0]; p.m_h = mask_str[1]; p.m_q = mask_str[2];
-  p.k_s = p.v_s = (D + 7) / 8 * 8;
-  p.mask_narrow = 1;  // the layout with the most use for it
-  cmpext3::MaskBits mb;
-  if (!cmpext3::mask_bits_applies(p, causal != 0) || cmpext3::decode16_applies(p, causal != 0) ||
-      !cmpext3::mask_bits_plan(p, &mb))
+  // rows in whole 16-byte chunks only (narrow rows read the mask as it is), and
+  // the mask's base at the alignment with the most use for the bits
+  if ((dtype != CMPEXT3_DTYPE_F16 && dtype != CMPEXT3_DTYPE_BF16) || mask_dtype != CMPEXT3_DTYPE_BOOL ||
+      !mask_str || !whole_chunks(dtype, D))
     return 0;
-  return mb.bytes + 256;  // the exchange in front of it ends anywhere
+  cmpext3::SplitInfo info;
+  if (plan_impl(dtype, B, H, H_kv, Sq, Sk, D, mask_dtype, causal, 0, 0, SIZE_MAX, info, mask_str) != CMPEXT3_OK ||
+      info.bits == 0)
+    return 0;
+  return info.bits + 256;  // the exchange in front of it ends anywhere
 }
 
 int cmpext3_attn_fwd_plan(int dtype, int B, int H, int H_kv, int Sq, int Sk, int D, int mask_dtype,

@@ -355,6 +355,7 @@ constexpr int64_t kMaskBitsMaxBytes = int64_t(128) << 20;
 struct SplitInfo {
   size_t need;
   int parts;
+  size_t bits = 0;  // bytes of the mask's bit form, where the launch makes one
 };
 
 // Bind a key-split plan to exchange space (host side, attn_fwd_plan16.hip).

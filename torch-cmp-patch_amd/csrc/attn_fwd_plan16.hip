@@ -441,6 +441,8 @@ hipError_t launch_pipe16(const FwdParams& p0, int dk0, bool bf16, bool causal, b
   if (p.dry) {
     // the size query reports the best plan's need (stream-K's, when it applies)
     if (sk_need > p.dry->need) p.dry->need = sk_need;
+    MaskBits mb;
+    if (mask_bits_applies(p, causal) && mask_bits_plan(p, &mb)) p.dry->bits = mb.bytes;
     return hipSuccess;
   }
   if (mask_bits_applies(p, causal)) {
