@@ -6,6 +6,7 @@ The library is loaded from this package directory; loading it needs no GPU.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from typing import Optional
@@ -123,18 +124,42 @@ def plan(dtype: int, B: int, H: int, Hkv: int, Sq: int, Sk: int, D: int, workspa
 _workspaces: dict = {}
 
 
-def workspace_for(t, handle: int, need: int):
-    """(pointer, bytes) of the workspace for stream `handle` on t's device, at
-    least `need` bytes; (None, 0) under graph capture or when need is 0."""
+# Mask bits are kept there up to KEPT_MASK_BITS, in steps; a larger mask's call
+# takes a workspace of its own.
+KEPT_MASK_BITS, WORKSPACE_STEP = 16 << 20, 4 << 20
+
+
+def workspace_for(t, handle: int, need: int, bits: int = 0):
+    """The workspace for stream `handle` on t's device, at least `need` bytes
+    plus `bits` of mask bits, or None (under graph capture, or when both are
+    0).  Hold it until the launch is made: another thread may replace the kept
+    one by a larger one meanwhile."""
     import torch
+    if bits:
+        need = max(need, WORKSPACE_COUNTER_BYTES) + bits
     if need == 0 or torch.cuda.is_current_stream_capturing():
-        return None, 0
+        return None
     key = (t.device.index, handle)
-    w = _workspaces.get(key)
-    if w is None or w.numel() < need:
-        w = torch.zeros(need, dtype=torch.uint8, device=t.device)
-        _workspaces[key] = w
-    return w.data_ptr(), w.numel()
+    keep = bits <= KEPT_MASK_BITS
+    w = _workspaces.get(key) if keep else None
+    if w is not None and w.numel() >= need:
+        return w
+    # made, cleared and given back in the order of the stream that uses it
+    same = handle == torch.cuda.current_stream(t.device).cuda_stream
+    with contextlib.nullcontext() if same else torch.cuda.stream(torch.cuda.ExternalStream(handle, device=t.device)):
+        if keep:
+            if bits:
+                need = (need + WORKSPACE_STEP - 1) // WORKSPACE_STEP * WORKSPACE_STEP
+            w = _workspaces[key] = torch.zeros(need, dtype=torch.uint8, device=t.device)
+        else:
+            w = torch.empty(need, dtype=torch.uint8, device=t.device)
+            w[:WORKSPACE_COUNTER_BYTES].zero_()
+    return w
+
+
+def _space(w):
+    """(pointer, bytes) of a workspace tensor or None."""
+    return (None, 0) if w is None else (w.data_ptr(), w.numel())
 
 
 def dtype_code(dtype) -> int:
@@ -196,13 +221,13 @@ def attn_fwd_raw(q, k, v, o, scale: float, causal: bool = False, stream=None,
             return lib().cmpext3_attn_fwd_gqa(*ptrs, dt, B, H, k.shape[1], Sq, k.shape[2], Dx, *tail)
         return lib().cmpext3_attn_fwd(*ptrs, dt, B, H, Sq, k.shape[2], Dx, *tail)
     mp, mdt, mst, _keep = _mask_args(attn_mask, B, H, Sq, k.shape[2])
-    wp, wb = None, 0
+    ws = None
     if workspace is True and q.is_cuda:
-        need = workspace_size(dt, B, H, k.shape[1], Sq, k.shape[2], Dx, mdt, causal)
-        bits = mask_workspace_size(dt, B, H, k.shape[1], Sq, k.shape[2], Dx, mdt, mst, causal)
-        wp, wb = workspace_for(q, handle, max(need, WORKSPACE_COUNTER_BYTES) + bits if bits else need)
-    elif workspace is not False and workspace is not None:
-        wp, wb = workspace.data_ptr(), workspace.numel()
+        ws = workspace_for(q, handle, workspace_size(dt, B, H, k.shape[1], Sq, k.shape[2], Dx, mdt, causal),
+                           mask_workspace_size(dt, B, H, k.shape[1], Sq, k.shape[2], Dx, mdt, mst, causal))
+    elif workspace is not True and workspace is not False:
+        ws = workspace
+    wp, wb = _space(ws)
     return lib().cmpext3_attn_fwd_ws(*ptrs, dt, B, H, k.shape[1], Sq, k.shape[2], Dx, *strides,
                                      mp, mdt, mst, ctypes.c_float(scale), int(causal),
                                      ctypes.c_void_p(wp), wb, ctypes.c_void_p(handle))
@@ -266,9 +291,9 @@ def attn_fwd_lse(q, k, v, scale: Optional[float] = None, causal: bool = False, s
         scale = D ** -0.5
     mp, mdt, mst, _keep = _mask_args(attn_mask, B, H, Sq, k.shape[2], runs=True)
     handle = _handle(q, stream)
-    wp, wb = workspace_for(q, handle, workspace_size(dtype_code(q.dtype), B, H, k.shape[1], Sq,
-                                                     k.shape[2], D, mdt, causal, with_lse=True)) \
-        if workspace else (None, 0)
+    ws = workspace_for(q, handle, workspace_size(dtype_code(q.dtype), B, H, k.shape[1], Sq, k.shape[2], D, mdt,
+                                                 causal, with_lse=True)) if workspace else None
+    wp, wb = _space(ws)
     rc = lib().cmpext3_attn_fwd_lse(
         ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(v.data_ptr()),
         ctypes.c_void_p(o.data_ptr()), ctypes.c_void_p(lse.data_ptr()), dtype_code(q.dtype),

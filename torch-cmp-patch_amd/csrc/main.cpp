@@ -75,15 +75,26 @@ struct Workspace {
 std::mutex ws_mu;
 std::map<std::pair<int, hipStream_t>, torch::Tensor> ws_cache;  // guarded by ws_mu
 
-Workspace workspace_for(const torch::Tensor& like, hipStream_t stream, size_t need) {
-  Workspace w;
-  if (need == 0) return w;
+// Mask bits (up to 128 MiB) share the kept workspace up to this size, in steps
+// of kWorkspaceStep so that prompts of rising length do not each make and clear
+// a new one; a larger mask's call takes a workspace of its own and gives it
+// back (cleared over its counters alone: microseconds, in a call that reads
+// over 100 MB of mask).
+constexpr size_t kKeptMaskBits = size_t(16) << 20;
+constexpr size_t kWorkspaceStep = size_t(4) << 20;
+
+bool capturing(hipStream_t stream) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
     (void)hipGetLastError();
-    return w;
+    return true;
   }
-  if (cap != hipStreamCaptureStatusNone) return w;
+  return cap != hipStreamCaptureStatusNone;
+}
+
+Workspace workspace_for(const torch::Tensor& like, hipStream_t stream, size_t need) {
+  Workspace w;
+  if (need == 0 || capturing(stream)) return w;
   std::lock_guard<std::mutex> lock(ws_mu);
   torch::Tensor& t = ws_cache[std::make_pair((int)like.get_device(), stream)];
   if (!t.defined() || (size_t)t.numel() < need)
@@ -117,7 +128,19 @@ int launch(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& 
   size_t need = cmpext3_attn_fwd_workspace_size(dtype, B, H, Hkv, Sq, Sk, D, mask.dtype, causal ? 1 : 0, 0);
   const size_t bits = cmpext3_attn_fwd_mask_workspace_size(dtype, B, H, Hkv, Sq, Sk, D, mask.dtype, ms, causal ? 1 : 0);
   if (bits > 0) need = std::max(need, (size_t)CMPEXT3_WORKSPACE_COUNTER_BYTES) + bits;
-  const Workspace ws = workspace_for(q, stream, need);
+  Workspace ws;
+  torch::Tensor own;  // freed on return: the allocator reuses it in stream order
+  if (bits > kKeptMaskBits) {
+    if (!capturing(stream)) {
+      own = torch::empty({(int64_t)need}, q.options().dtype(at::kByte));
+      own.narrow(0, 0, CMPEXT3_WORKSPACE_COUNTER_BYTES).zero_();
+      ws.ptr = own.data_ptr();
+      ws.bytes = need;
+    }
+  } else {
+    if (bits > 0) need = (need + kWorkspaceStep - 1) / kWorkspaceStep * kWorkspaceStep;
+    ws = workspace_for(q, stream, need);
+  }
   return cmpext3_attn_fwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dtype, B, H, Hkv, Sq,
                              Sk, D, qs, ks, vs, os, mask.dtype >= 0 ? mask.t.data_ptr() : nullptr,
                              mask.dtype, ms, scale, causal ? 1 : 0, ws.ptr, ws.bytes, stream);
