@@ -140,6 +140,10 @@ int cmpext3_attn_fwd_gqa(const void* q, const void* k, const void* v, void* o,
  *                multiple of 8 the keys are read in runs of 8; any other
  *                layout element by element.)
  * A query row whose keys are all dropped gives zeros (torch's result).
+ * A dropped key has weight 0, and 0 times an infinity or NaN in V is NaN (as
+ * in torch's math): such a value at a dropped key may reach a row's output.
+ * Which rows it reaches is not specified: a launch leaves out whole tiles of
+ * keys that none of its block's rows keep (causal; bool masks in bit form).
  * With causal != 0 a pair is used only if it is causally visible AND the
  * mask keeps it (torch's rule for attn_mask with is_causal).  Supported for
  * every dtype (f16, bf16, f32) and head dim; the rows of q/k/v/o must be

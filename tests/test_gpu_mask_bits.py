@@ -13,6 +13,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+import cmpext3
 from cmpext3 import abi
 from cmpext3 import workloads as W
 from oracle import sdpa_oracle as orc
@@ -102,6 +103,42 @@ def test_allocation_free_entry_point_makes_the_bits_too():
     assert abi.attn_fwd_raw(q, k, v, b, 0.125, attn_mask=m, workspace=ws) == 0
     torch.cuda.synchronize()
     assert torch.equal(a, b)
+
+
+def _tell_tale(dtype, Sq, Sk, D):
+    """Inputs whose result says whether the bits were made: V is NaN over key
+    tiles that no query keeps.  The bit form leaves those tiles out; the mask
+    read as it is weighs them 0, and 0 * NaN is NaN."""
+    q, k, v = W.Workload("bt", dtype, 2, 4, Sq, Sk, D, seed=Sk).make_inputs("cuda")
+    m = _mask("left_pad", 2, 4, Sq, Sk, 0) & (torch.arange(Sk) // 32 != 2)
+    m |= torch.arange(Sk) < 8  # every row keeps a key
+    nan = v.clone()
+    nan[:, :, 64:96] = float("nan")
+    keep = m.expand(2, 4, Sq, Sk)
+    return q, k, nan, m.cuda(), orc.sdpa_np(q.cpu(), k.cpu(), v.cpu(), D ** -0.5, False, attn_mask=keep)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,Sq,Sk,D", [("fp16", 300, 777, 64), ("bf16", 300, 776, 128), ("bf16", 520, 1001, 128),
+                                           ("fp16", 300, 600, 192)])
+@pytest.mark.parametrize("side", ["abi", "given workspace", "allocation-free", "binding"])
+def test_the_bits_are_made(dtype, Sq, Sk, D, side):
+    q, k, v, m, want = _tell_tale(dtype, Sq, Sk, D)
+    out = torch.empty_like(q)
+    if side == "abi":
+        assert abi.attn_fwd_raw(q, k, v, out, D ** -0.5, False, attn_mask=m) == 0
+    elif side == "given workspace":
+        ws = torch.zeros(16 << 20, dtype=torch.uint8, device="cuda")
+        assert abi.attn_fwd_raw(q, k, v, out, D ** -0.5, False, attn_mask=m, workspace=ws) == 0
+    elif side == "allocation-free":
+        assert abi.attn_fwd_noalloc_raw(q, k, v, out, D ** -0.5, False, attn_mask=m) == 0
+    else:
+        out = cmpext3.ops.attention(q, k, v, None, False, m)
+    as_it_is = torch.empty_like(q)
+    assert abi.attn_fwd_raw(q, k, v, as_it_is, D ** -0.5, False, attn_mask=m, workspace=False) == 0
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all() and orc.max_abs_err(out.cpu(), want) <= TOL[dtype]
+    assert torch.isnan(as_it_is).any()  # the inputs do tell the two apart
 
 
 def test_mask_workspace_size():
