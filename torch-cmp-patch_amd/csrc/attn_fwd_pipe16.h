@@ -1064,8 +1064,11 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     };
     auto weight = [&](float m) { return m == -INFINITY ? 0.f : fast_exp2(m - moff); };
     float lnew = 0.f;
-    if (half_x && nparts == 2) {
-      // O / l in fp16, weighted by a * l: the other part's all at once
+    if (half_x && nparts == 2 && NDB <= 4) {
+      // O / l in fp16, weighted by a * l: the other part's all at once.  (Above
+      // D = 128 they do not fit beside the accumulators: part by part below,
+      // fp16 [1,12,1024,1024,256] 35.5 us against 37.2, [1,16,777,777,256] 31.5
+      // against 33.3.)
       u32x4 x[2 * NDB];
       const f32x2 mo = ml_of(1 - part);
 #pragma unroll
