@@ -24,7 +24,7 @@ CASES = [
     (1, 8, 2048, 64, False, False),
     (1, 10, 4096, 64, False, False),
     (1, 20, 2048, 64, False, False),     # the tail of whole rounds
-    (1, 8, 2048, 64, True, False),
+    (1, 12, 2048, 64, True, False),
     (1, 16, 2048, 64, True, True),
     (1, 10, 1024, 128, False, False),
     (1, 2, 448, 256, False, True),       # fewer key tiles than two parts usually want

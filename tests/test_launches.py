@@ -173,3 +173,15 @@ print(json.dumps(out))
     assert len(got) > 300 and any(size for *_, size, _ in got)
     for *case, rc, size, made in got:
         assert rc == 0 and (size > 0) == (made == 1), (case, size, made)
+
+
+@pytest.mark.parametrize("H,S,D,parts", [
+    (2, 1024, 64, 2), (2, 2048, 64, 4), (2, 2048, 256, 4), (4, 2048, 128, 4), (6, 2048, 64, 3),
+    (8, 2048, 64, 3), (8, 3072, 64, 3), (2, 6000, 64, 4), (12, 2048, 64, 2), (16, 2048, 64, 2),
+    (32, 1024, 128, 1)])
+def test_small_causal_grids_keep_a_part_per_cu(H, S, D, parts):
+    import torch
+    from cmpext3 import abi
+    if torch.cuda.is_available():
+        pytest.skip("plan depends on the visible device's CU count")
+    assert abi.plan(abi.DTYPE_BF16, 1, H, H, S, S, D, 1 << 40, causal=True) == (abi.OK, parts)

@@ -115,8 +115,9 @@ float cut_cost(int dk, bool half, int n) {
 // Parts of every block of a non-causal prefill with fewer blocks than CUs
 // (half: two of them exchange in fp16).
 // With a part to a CU, P parts save nt (1 - 1/P) tiles; two parts beyond that
-// share CUs and save 0.38 nt (above D = 128 a CU holds one workgroup: nothing).  Three parts and more all leave fp32 states, and
-// from four on a launch pays another 5 (D > 128) or 12 tiles: bf16
+// share CUs and save 0.38 nt (above D = 128 a CU holds one workgroup: nothing).
+// Three parts and more all leave fp32 states, and from four on a launch pays
+// another 5 (D > 128) or 12 tiles: bf16
 // [1,8,1024,1024,D], 64 blocks, whole / in 2 / 3 / 4 parts, D = 64: 16.1 / 13.8
 // / 12.8 / 17.2 us, D = 128: 21.5 / 19.9 / 19.4 / 23.1, D = 256: 46.7 / 37.5 /
 // 34.3 / 37.1.
@@ -154,11 +155,16 @@ int prefill_parts(int dk, bool half, int n, int nt, int cus, int occ) {
 // prologues and merges ([1,32,1024,128] 25 -> 28 us, [1,32,512,128] 16 ->
 // 18 us) and stay whole.  More than two parts want longer ones
 // (kMinManyCausalTiles: bf16 [1,16,2048,64] 29.2 whole, 23.1 in 2, 26.7 in 3;
-// [1,8,2048,128] 39.2 / 27.1 / 27.9, 35.3 in 4), and beyond the smallest
-// grids more than three lose ([1,8,3072,64] 25.3 in 3, 32.1 in 4).  Every part
-// of every block keeps at least one tile
-// (a causal row sees a key in the first tile of a part, or none of the part's
-// keys: its state then has no weight in the merge).
+// [1,8,2048,128] 39.2 / 27.1 / 27.9, 35.3 in 4), and where four would fill more
+// than 3/4 of the slots three are better ([1,8,3072,64] 25.3 in 3, 32.1 in 4;
+// below that [1,2,6000,64] 32.3 in 3, 28.9 in 4).  Where the
+// parts still have a CU each, shorter ones pay as well ([1,2,2048,64] 19.2 in
+// 2, 14.7 in 4; [1,4,2048,128] 26.1 / 21.3; [1,2,2048,256] 52.8 / 38.3), and at
+// three workgroups per CU three parts of up to half as many blocks as CUs
+// ([1,6,2048,64] 19.8 in 2, 17.3 in 3, 18.5 in 4; [1,8,2048,64] 20.0 / 17.8).
+// Every part of every block keeps at least one tile (a causal row sees a key in
+// the first tile of a part, or none of the part's keys: its state then has no
+// weight in the merge).
 SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntiles_min, const PlanKind& k) {
   SplitArgs sa = {n, 1, nullptr, nullptr, kPipeNw};
   if (cus <= 0) return sa;
@@ -172,7 +178,11 @@ SplitArgs split_plan(int n, int ntiles, int occ, int cus, bool causal, int ntile
     int parts = most;
     if (parts > 2 && parts > ntiles / kMinManyCausalTiles)
       parts = ntiles / kMinManyCausalTiles > 2 ? ntiles / kMinManyCausalTiles : 2;
-    if (parts > 3 && n * 3 > cus) parts = 3;
+    if (parts > 3 && n * 16 > slots * 3) parts = 3;
+    int own = cus / n;  // parts that have a CU each
+    if (occ >= 3 && own < 3 && n * 2 <= cus) own = 3;
+    if (own > most) own = most;
+    if (parts < own) parts = own;
     if (parts < 2) return sa;
     sa.nfull = 0;
     sa.nparts = parts;
