@@ -304,12 +304,15 @@ int cmpext3_attn_fwd_lse(const void* q, const void* k, const void* v, void* o, f
  *   delta : caller-owned fp32 workspace of B*H*Sq elements (4-byte aligned;
  *           receives sum_d dout * o per row).
  *   *_str[3] : element strides over {batch, head, seq} as in cmpext3_attn_fwd.
- * Three kernels on `stream`: Delta, dK/dV (one workgroup per 128 keys of a
- * K/V head; 64 for fp32), dQ (one per 128 queries; 64 for fp32); each
- * gradient row is written by exactly one workgroup, so results are
- * bit-identical from run to run.  This entry point takes no workspace and
- * never splits a sweep (cmpext3_attn_bwd_ws below can).  B*H*Sq == 0 is a no-op (dk and dv are then
- * left untouched).  Every dtype: f16/bf16 on 32x32x16 MFMAs (head dims above
+ * Two kernels on `stream`: Delta, then both gradients in one launch, whose
+ * workgroups sweep dK/dV (one per 128 keys of a K/V head; 64 for fp32) or dQ
+ * (one per 128 queries; 64 for fp32).  A few forms (masked causal grids at
+ * D <= 64 that fill the chip, more than 2^32 threads together) launch the two
+ * sweeps one after the other.  Each gradient row is written by exactly one
+ * workgroup, so results are bit-identical from run to run.  This entry point
+ * takes no workspace and never splits a sweep (cmpext3_attn_bwd_ws below can,
+ * and then sums the parts in further launches).  B*H*Sq == 0 is a no-op (dk
+ * and dv are then left untouched).  Every dtype: f16/bf16 on 32x32x16 MFMAs (head dims above
  * 128 in the 192 and 256 buckets at one wave per SIMD), fp32 on 16x16x4 fp32
  * MFMAs (buckets 32, 40, 64, 96, 128, 192, 256).
  *

@@ -15,9 +15,13 @@
 // one row for all queries has one block.  Both arrays live in the caller's
 // workspace behind the key split's exchange, rewritten by every call.
 //
-// Bound: the mask's bytes from HBM, once.  bf16 [4,16/8,1531,1531,128] with a
-// bool [B,1,Sq,Sk] mask, causal and left-padded: 492 us with the mask read by
-// the element, 61 us with this pass and the tiles it lets the sweep skip.
+// Bound: latency, not bytes.  A lane holds one row, so a load touches 64 lines,
+// and a last tile that is not whole is read byte by byte in a loop: 13.7 us for
+// the 9.4 MB of a [4,1,1531,1531] mask (0.7 TB/s, a seventh of a copy's rate),
+// of which the last tile has 27 single bytes per row.  Small beside what it
+// saves: bf16 [4,16/8,1531,1531,128] with that mask, causal and left-padded,
+// 492 us with the mask read by the element, 61 us with this pass and the tiles
+// it lets the sweep skip.
 #include "attn_common.h"
 
 namespace cmpext3 {
