@@ -331,10 +331,11 @@ struct TileLoader {
   // soff: byte offset of the tile's first row, below range
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t range, int soff, u32x4 (&x)[N]) const {
 #pragma unroll
-    for (int it = 0; it < N; ++it)
+    for (int it = 0; it < N; ++it) {
+      const int so = BYROW && it > 0 ? (int)min((uint32_t)soff + (uint32_t)(it * step), range) : soff;
       x[it] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, BYROW ? voff : voff + 128 * it,
-                                                       BYROW && it > 0 ? (int)min((uint32_t)(soff + it * step), range) : soff, 0));
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, BYROW ? voff : voff + 128 * it, so, 0));
+    }
   }
   template <int RS>
   __device__ __forceinline__ void store(uint16_t* dst, const u32x4 (&x)[N]) const {

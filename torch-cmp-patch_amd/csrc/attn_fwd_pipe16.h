@@ -975,9 +975,10 @@ __device__ __forceinline__ void pipe16_segment(const FwdParams& p, const SplitAr
     const float m_own = lsum > 0.f ? mb : -INFINITY;
     // Two fp16 parts, where the plan says so (short blocks: always), exchange
     // their O normalised by their own row sum, in fp16 (half of the bytes):
-    // 2 * NDB vectors, then (m, l) as 8 bytes per lane.  Both parts round their own O this way, so the result does
-    // not depend on which one writes (reruns stay bit-identical); rounding O/l
-    // to fp16 before the merge adds at most one fp16 rounding to the output.
+    // 2 * NDB vectors, then (m, l) as 8 bytes per lane.  Both parts round their
+    // own O this way, so the result does not depend on which one writes (reruns
+    // stay bit-identical); rounding O/l to fp16 before the merge adds at most
+    // one fp16 rounding to the output.
     const bool half_x = std::is_same<T, _Float16>::value && (STREAMK || (nparts == 2 && ((OPT & 128) || sa.half16)));
     u32x4 own_h[2 * NDB];  // half_x: this part's O / l in fp16
     if (half_x) {

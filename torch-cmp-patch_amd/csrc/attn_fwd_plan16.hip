@@ -151,17 +151,17 @@ int prefill_parts(int dk, bool half, int n, int nt, int cus, int occ) {
 // kMinCausalPartTiles tiles: each block's longest part, and so the launch,
 // gets shorter.  Measured on MI355X (same run): [1,4,8192,128] bf16 135 ->
 // 98 us, [1,8,2048,256] 85 -> 54 us, [1,8,1024,64] 17.2 -> 13.8 us; shorter
-// sweeps on busy CUs lost to the parts'
-// prologues and merges ([1,32,1024,128] 25 -> 28 us, [1,32,512,128] 16 ->
-// 18 us) and stay whole.  More than two parts want longer ones
-// (kMinManyCausalTiles: bf16 [1,16,2048,64] 29.2 whole, 23.1 in 2, 26.7 in 3;
-// [1,8,2048,128] 39.2 / 27.1 / 27.9, 35.3 in 4), and where four would fill more
-// than 3/4 of the slots three are better ([1,8,3072,64] 25.3 in 3, 32.1 in 4;
-// below that [1,2,6000,64] 32.3 in 3, 28.9 in 4).  Where the
-// parts still have a CU each, shorter ones pay as well ([1,2,2048,64] 19.2 in
-// 2, 14.7 in 4; [1,4,2048,128] 26.1 / 21.3; [1,2,2048,256] 52.8 / 38.3), and at
-// three workgroups per CU three parts of up to half as many blocks as CUs
-// ([1,6,2048,64] 19.8 in 2, 17.3 in 3, 18.5 in 4; [1,8,2048,64] 20.0 / 17.8).
+// sweeps on busy CUs lost to the parts' prologues and merges
+// ([1,32,1024,128] 25 -> 28 us, [1,32,512,128] 16 -> 18 us) and stay whole.
+// More than two parts want longer ones (kMinManyCausalTiles: bf16
+// [1,16,2048,64] 29.2 whole, 23.1 in 2, 26.7 in 3; [1,8,2048,128] 39.2 / 27.1 /
+// 27.9, 35.3 in 4), and where four would fill more than 3/4 of the slots three
+// are better ([1,8,3072,64] 25.3 in 3, 32.1 in 4; below that [1,2,6000,64] 32.3
+// in 3, 28.9 in 4).  Where the parts still have a CU each, shorter ones pay as
+// well ([1,2,2048,64] 19.2 in 2, 14.7 in 4; [1,4,2048,128] 26.1 / 21.3;
+// [1,2,2048,256] 52.8 / 38.3), and at three workgroups per CU three parts of up
+// to half as many blocks as CUs ([1,6,2048,64] 19.8 in 2, 17.3 in 3, 18.5 in 4;
+// [1,8,2048,64] 20.0 / 17.8).
 // Every part of every block keeps at least one tile (a causal row sees a key in
 // the first tile of a part, or none of the part's keys: its state then has no
 // weight in the merge).
