@@ -31,6 +31,6 @@ def test_backward_kernels_keep_their_parameters_in_registers():
             dk, sweep = int(f32[1]), int(f32[2])
             tiles = 2 * 2 * 32 * ((dk + 15) // 16 * 16 + 4) * 4  # [slot][operand][row][col]
             assert k[".private_segment_fixed_size"] == 0, name
-            assert k[".group_segment_fixed_size"] == tiles + (16 if sweep == 2 else 512), name
+            assert k[".group_segment_fixed_size"] == tiles + (0 if sweep == 2 else 512), name
             seen += 1
     assert seen >= 16
