@@ -27,10 +27,15 @@ def test_backward_kernels_keep_their_parameters_in_registers():
     seen = 0
     for name, k in _kernels(abi.LIB_PATH).items():
         f32 = re.search(r"attn_bwd32_gradsILi(\d+)ELb\dELi(\d)E", name)
+        f16 = re.search(r"attn_bwd_gradsIDF16b?_?Li(\d+)ELb(\d)ELb(\d)ELi\dE", name)
         if f32:
             dk, sweep = int(f32[1]), int(f32[2])
             tiles = 2 * 2 * 32 * ((dk + 15) // 16 * 16 + 4) * 4  # [slot][operand][row][col]
             assert k[".private_segment_fixed_size"] == 0, name
             assert k[".group_segment_fixed_size"] == tiles + (0 if sweep == 2 else 512), name
-            seen += 1
-    assert seen >= 16
+        elif f16:
+            # masked, not causal, D <= 64 spills a few registers for its third wave
+            spills = (int(f16[1]), f16[2], f16[3]) == (64, "0", "1")
+            assert k[".private_segment_fixed_size"] <= (20 if spills else 0), name
+        seen += bool(f32 or f16)
+    assert seen >= 40

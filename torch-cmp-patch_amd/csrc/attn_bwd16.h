@@ -441,7 +441,7 @@ struct BwdDkdv {
 
 // Workgroup `wg` of the dK/dV sweeps; its LDS arrays (BwdDkdv's sizes).
 template <typename T, int DK, bool CAUSAL, bool MASK>
-__device__ __forceinline__ void bwd_dkdv_block(const BwdParams& p, const int wg, uint16_t* const lds,
+__device__ __forceinline__ void bwd_dkdv_block(const BwdParams p, const int wg, uint16_t* const lds,
                                                uint16_t* const vpark, float* const lsdp) {
   using Cfg = BwdDkdv<DK, CAUSAL, MASK>;
   constexpr int BQ = Cfg::BQ, BKV = Cfg::BKV, RS = Cfg::RS, KP = Cfg::KP;
@@ -847,7 +847,7 @@ struct BwdDq {
 
 // Workgroup `wg` of the dQ sweeps; its LDS arrays (BwdDq's sizes).
 template <typename T, int DK, bool CAUSAL, bool MASK>
-__device__ __forceinline__ void bwd_dq_block(const BwdParams& p, const int wg, uint16_t* const lds,
+__device__ __forceinline__ void bwd_dq_block(const BwdParams p, const int wg, uint16_t* const lds,
                                              uint16_t* const dpark) {
   using Cfg = BwdDq<DK, CAUSAL, MASK>;
   constexpr int BQ = Cfg::BQ, BK = Cfg::BK, RS = Cfg::RS, RSD = Cfg::RSD;
